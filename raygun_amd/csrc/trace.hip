@@ -16,10 +16,11 @@ constexpr int kSpill = 368; // with the 16 LDS entries: the 381-entry worst case
 // Wavefront trace pass: rays [0, count) of queue `cur` -> hit records.
 // Waves fetch 64 rays at a time from a global counter (persistent grid).
 // Waves per SIMD the traversal pass is compiled for: the register budget is
-// 512 / waves VGPRs (7: 73, which its 71 fit without spilling; more waves
-// hide more of the node-fetch latency; 8 spills).
+// 512 / waves VGPRs. At 7 waves (73) nine registers spill in the loop: a
+// 1080p frame over 2M triangles takes 8.92 ms against 8.75 at 6 waves, 3,000
+// small instances 3.74 against 3.62 ms.
 #ifndef RGRT_TRACE_WAVES
-#define RGRT_TRACE_WAVES 7
+#define RGRT_TRACE_WAVES 6
 #endif
 
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(RGRT_TRACE_WAVES))) void k_trace_queue(TraceScene sc, const float* __restrict__ rays,
@@ -61,7 +62,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(RGR
             r.dz = rays[6 * (size_t)npix + i];
             r.tmax = rays[7 * (size_t)npix + i];
             const uint32_t flags = __float_as_uint(rays[9 * (size_t)npix + i]);
-            const HitRec h = traverse<RGRT_INST_EVERY, RGRT_TRI_EVERY, RGRT_SENT_EVERY>(sc, r, (flags >> kMaskShift) & 0xffu, stack);
+            const HitRec h = traverse<RGRT_INST_EVERY>(sc, r, (flags >> kMaskShift) & 0xffu, stack);
             hits[0 * (size_t)npix + i] = h.t;
             hits[1 * (size_t)npix + i] = h.u;
             hits[2 * (size_t)npix + i] = h.v;
@@ -139,7 +140,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(RGR
             r.dz = rays[6 * npix + i];
             r.tmax = rays[7 * npix + i];
             const uint32_t flags = __float_as_uint(rays[9 * npix + i]);
-            const HitRec h = traverse<RGRT_INST_EVERY, RGRT_TRI_EVERY, RGRT_SENT_EVERY>(sc, r, (flags >> kMaskShift) & 0xffu, stack);
+            const HitRec h = traverse<RGRT_INST_EVERY>(sc, r, (flags >> kMaskShift) & 0xffu, stack);
             hits[0 * npix + i] = h.t;
             hits[1 * npix + i] = h.u;
             hits[2 * npix + i] = h.v;
@@ -166,7 +167,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_rays(TraceScene sc, const
     for(uint32_t i = gtid; i < n; i += gridDim.x * kTraceBlock) {
         const rgrt_ray rr = rays[i];
         RayIn r{rr.origin[0], rr.origin[1], rr.origin[2], rr.tmin, rr.dir[0], rr.dir[1], rr.dir[2], rr.tmax};
-        const HitRec h = traverse<RGRT_INST_EVERY, RGRT_TRI_EVERY, RGRT_SENT_EVERY>(sc, r, cullMask & 0xffu, stack);
+        const HitRec h = traverse<RGRT_INST_EVERY>(sc, r, cullMask & 0xffu, stack);
         rgrt_hit o;
         o.t = h.t;
         o.u = h.u;

@@ -98,10 +98,9 @@ __device__ __forceinline__ float qbox_enter(uint32_t nx, uint32_t fx, uint32_t n
 // children but the nearest farthest first and returns the nearest
 // (kEmptyChild if none was hit).
 template<typename Stack>
-__device__ __forceinline__ int32_t visit_wide(const Node4q* nodes, int32_t ref, const BoxRay& br, float tmin, float tbest, Stack& stack)
+__device__ __forceinline__ int32_t visit_wide(const u32x4 v0, const u32x4 v1, const u32x4 v2, const u32x4 v3, const BoxRay& br,
+                                              float tmin, float tbest, Stack& stack)
 {
-    const u32x4* np = reinterpret_cast<const u32x4*>(nodes + ref);
-    const u32x4 v0 = ld_global16(np), v1 = ld_global16(np + 1), v2 = ld_global16(np + 2), v3 = ld_global16(np + 3);
     const int4 ch = make_int4((int)v3.x, (int)v3.y, (int)v3.z, (int)v3.w);
     const int ex = (int)(int8_t)(v0.w & 0xffu), ey = (int)(int8_t)((v0.w >> 8) & 0xffu), ez = (int)(int8_t)((v0.w >> 16) & 0xffu);
     const float ax = pow2i(ex) * br.ix, ay = pow2i(ey) * br.iy, az = pow2i(ez) * br.iz;
@@ -144,14 +143,13 @@ __device__ __forceinline__ int32_t visit_wide(const Node4q* nodes, int32_t ref, 
 // symmetric), so t, u, v and the accept decision are the same without it.
 // The triangle copy `rot` = kz holds the vertices in (kx, ky, kz) order.
 struct WtRay {
-    int rot;
     float Sx, Sy, Sz;
     float okx, oky, okz; // origin in (kx, ky, kz) order
 };
 
 __device__ __forceinline__ float sel3(float x, float y, float z, int k) { return k == 0 ? x : (k == 1 ? y : z); }
 
-__device__ __forceinline__ void wt_setup(WtRay& w, float ox, float oy, float oz, float dx, float dy, float dz)
+__device__ __forceinline__ int wt_setup(WtRay& w, float ox, float oy, float oz, float dx, float dy, float dz)
 {
     int kz = 0;
     float m = fabsf(dx);
@@ -162,7 +160,6 @@ __device__ __forceinline__ void wt_setup(WtRay& w, float ox, float oy, float oz,
     if(fabsf(dz) > m) kz = 2;
     const int kx = kz + 1 == 3 ? 0 : kz + 1;
     const int ky = kx + 1 == 3 ? 0 : kx + 1;
-    w.rot = kz;
     const float dkz = sel3(dx, dy, dz, kz);
     const float dkx = sel3(dx, dy, dz, kx), dky = sel3(dx, dy, dz, ky);
     w.Sz = 1.0f / dkz; // one division; the shears reuse it
@@ -171,6 +168,7 @@ __device__ __forceinline__ void wt_setup(WtRay& w, float ox, float oy, float oz,
     w.okx = sel3(ox, oy, oz, kx);
     w.oky = sel3(ox, oy, oz, ky);
     w.okz = sel3(ox, oy, oz, kz);
+    return kz;
 }
 
 // Watertight ray/triangle test on a triangle copy in the ray's axis order;
@@ -287,14 +285,15 @@ struct Traversal {
     RayIn ray;
     float wix, wiy, wiz; // 1/d of the world ray (safe_rcp)
     WtRay wt;
-    const Node4q* nodes;
-    const Tri* tris;
+    const char* nodes;  // wide nodes of the tree being walked
+    const char* leaves; // its leaf records: instances or triangles
     float tbest;
     int32_t ref;
     uint32_t cullMask;
     uint32_t curInst;
-    uint32_t nodeCap;  // nodes of the tree being walked
-    uint32_t numFaces; // triangles of the BLAS being walked
+    uint32_t nodeCap;    // nodes of the tree being walked
+    uint32_t leafCap;    // its leaves
+    uint32_t leafStride; // bytes of a leaf record
     bool inBlas;
     HitRec h;
 };
@@ -303,6 +302,16 @@ struct Traversal {
 // indexes; a bad one (a corrupt tree or table) ends the ray as a miss and
 // raises a sticky flag that the host turns into an error.
 __device__ __noinline__ void trav_error(const TraceScene& sc, uint32_t flag) { atomicOr(sc.errors, flag); }
+
+__device__ __forceinline__ void enter_tlas(Traversal& T, const TraceScene& sc)
+{
+    T.nodes = reinterpret_cast<const char*>(sc.tlasNodes);
+    T.leaves = reinterpret_cast<const char*>(sc.instances);
+    T.nodeCap = sc.tlasNodeCap;
+    T.leafCap = sc.numInstances;
+    T.leafStride = sizeof(DevInstance);
+    T.inBlas = false;
+}
 
 // Starts a ray at the TLAS root; false if there is nothing to traverse.
 template<typename Stack>
@@ -313,15 +322,11 @@ __device__ __forceinline__ bool trav_begin(Traversal& T, const TraceScene& sc, c
     T.h.v = 0.0f;
     T.h.inst = kNoHit;
     T.h.prim = 0;
-    T.nodes = sc.tlasNodes;
-    T.tris = nullptr;
-    T.inBlas = false;
+    enter_tlas(T, sc);
     T.curInst = 0;
     T.tbest = ray.tmax;
     T.ref = 0;
     T.cullMask = cullMask;
-    T.nodeCap = sc.tlasNodeCap;
-    T.numFaces = 0;
     stack.sp = 0;
     T.wix = safe_rcp(ray.dx);
     T.wiy = safe_rcp(ray.dy);
@@ -330,104 +335,60 @@ __device__ __forceinline__ bool trav_begin(Traversal& T, const TraceScene& sc, c
     return sc.numInstances != 0;
 }
 
-// One step: a wide node, a sentinel, an instance leaf or a triangle.
+// One iteration of a wave's loop: a wide node, a triangle or an instance
+// leaf, and the pop after it, which takes the return to the TLAS with it.
 // Returns false once the ray is finished (T.h holds the closest hit).
 //
-// A wave runs every kind of step its lanes need in each iteration, so the
-// rare kinds (instance entry, triangle test) cost their instructions in
-// nearly every iteration. With kInstEvery / kTriEvery > 1 those steps are
-// taken only in iterations `iter` that are multiples of it; a lane that
-// reaches one in another iteration waits (its state is unchanged), which
-// delays that ray by a few iterations but leaves the wave's other
-// iterations without the path. Results do not change: every ray takes the
-// same steps in the same order. `iter` must count the wave's iterations
-// (all lanes start the ray together).
-template<int kInstEvery = 1, int kTriEvery = 1, int kSentEvery = 1, typename Stack>
+// A wave runs every kind of step its lanes need in each iteration and, if
+// each kind loads its own record, waits for one memory latency after the
+// other. So the record is fetched first, by the same four 16-byte loads
+// whatever the lane is at (a triangle's 48 bytes with the next 16, which
+// every triangle array has room for): one latency per iteration. On 1M
+// incoherent rays over 64 instances of 100k-triangle meshes 0.735 -> 0.640 ms
+// (pipelined), on a 1080p frame over 2M triangles 9.42 -> 8.75 ms. Running
+// an entry, the entered root, the triangle a node leads to and the pop in
+// one iteration, each with its own loads, needs a fifth fewer iterations
+// and was slower on those (0.687, 9.41 ms).
+//
+// An instance entry is rare (some 8% of a ray's steps) and costs as much as
+// a node visit, so it is taken only in iterations `iter` that are multiples
+// of kInstEvery; a lane that reaches one in another iteration waits with its
+// state unchanged. `iter` must count the wave's iterations (all lanes start
+// the ray together). Every ray takes the same steps in the same order
+// whatever kInstEvery is. Measured on the frame and the rays above: every
+// iteration 9.62 and 0.672 ms, every second 8.92 and 0.640, every fourth
+// 8.78 and 0.638; 3,000 small instances 4.08, 3.74 and 3.76 ms.
+template<int kInstEvery = 1, typename Stack>
 __device__ __forceinline__ bool trav_step(Traversal& T, const TraceScene& sc, Stack& stack, uint32_t iter = 0)
 {
-    if(T.ref >= 0) {
-        if((uint32_t)T.ref >= T.nodeCap) {
-            trav_error(sc, kTravErrNode);
-            T.h.inst = kNoHit;
-            return false;
-        }
-        const int32_t nearest = visit_wide(T.nodes, T.ref, stack.box_ray(), T.ray.tmin, T.tbest, stack);
-        if(nearest != kEmptyChild) {
-            T.ref = nearest;
-            return true;
-        }
+    const bool isNode = T.ref >= 0;
+    if(kInstEvery > 1 && iter % kInstEvery != 0u && !isNode && !T.inBlas) return true; // an entry of a later iteration
+    const uint32_t idx = (uint32_t)(isNode ? T.ref : ~T.ref);
+    if(idx >= (isNode ? T.nodeCap : T.leafCap)) {
+        trav_error(sc, isNode ? kTravErrNode : T.inBlas ? kTravErrTriangle : kTravErrInstance);
+        T.h.inst = kNoHit;
+        return false;
     }
-    else if(T.ref == kSentinel) {
-        if(kSentEvery > 1 && iter % kSentEvery != 0u) return true; // taken in a later iteration
-        T.inBlas = false;
-        T.nodes = sc.tlasNodes;
-        T.nodeCap = sc.tlasNodeCap;
-        stack.set_box_ray(T.ray.ox, T.ray.oy, T.ray.oz, T.wix, T.wiy, T.wiz);
+    // one fetch for whatever the lane is at
+    const u32x4* ip = reinterpret_cast<const u32x4*>((isNode ? T.nodes : T.leaves) + (uint64_t)idx * (isNode ? 64u : T.leafStride));
+    const u32x4 v0 = ld_global16(ip), v1 = ld_global16(ip + 1), v2 = ld_global16(ip + 2), v3 = ld_global16(ip + 3);
+    bool pop = true;
+    if(isNode) {
+        T.ref = visit_wide(v0, v1, v2, v3, stack.box_ray(), T.ray.tmin, T.tbest, stack);
+        pop = T.ref == kEmptyChild;
     }
-    else if(!T.inBlas) {
-        if(kInstEvery > 1 && iter % kInstEvery != 0u) return true; // taken in a later iteration
-        const int32_t leaf = ~T.ref;
-        if((uint32_t)leaf >= sc.numInstances) {
-            trav_error(sc, kTravErrInstance);
-            T.h.inst = kNoHit;
-            return false;
-        }
-        const u32x4* ip = reinterpret_cast<const u32x4*>(sc.instances + leaf);
-        const u32x4 i3 = ld_global16(ip + 3); // blas, mask, position, customIndex
-        if(i3.x >= sc.numBlas) {
-            trav_error(sc, kTravErrBlas);
-            T.h.inst = kNoHit;
-            return false;
-        }
-        const u32x4* bp = reinterpret_cast<const u32x4*>(sc.blas + i3.x);
-        const u32x4 b0 = ld_global16(bp);     // nodes, tris
-        const uint32_t numFaces = ld_global8(bp + 1).x;
-        if((i3.y & T.cullMask) != 0u && numFaces > 0u) {
-            float w[12];
-            for(int q = 0; q < 3; ++q) {
-                const u32x4 r = ld_global16(ip + q);
-                w[4 * q + 0] = __uint_as_float(r.x);
-                w[4 * q + 1] = __uint_as_float(r.y);
-                w[4 * q + 2] = __uint_as_float(r.z);
-                w[4 * q + 3] = __uint_as_float(r.w);
-            }
-            float rox, roy, roz, rdx, rdy, rdz;
-            xform_ray(w, T.ray.ox, T.ray.oy, T.ray.oz, T.ray.dx, T.ray.dy, T.ray.dz, rox, roy, roz, rdx, rdy, rdz);
-            stack.set_box_ray(rox, roy, roz, safe_rcp(rdx), safe_rcp(rdy), safe_rcp(rdz));
-            wt_setup(T.wt, rox, roy, roz, rdx, rdy, rdz);
-            stack.push(kSentinel);
-            T.nodes = reinterpret_cast<const Node4q*>((uint64_t)b0.x | ((uint64_t)b0.y << 32));
-            // the copy of the triangles in this ray's axis order
-            T.tris = reinterpret_cast<const Tri*>((uint64_t)b0.z | ((uint64_t)b0.w << 32)) + (size_t)T.wt.rot * numFaces;
-            T.inBlas = true;
-            T.curInst = i3.z;
-            T.numFaces = numFaces;
-            T.nodeCap = numFaces > 2u ? numFaces - 1u : 1u;
-            T.ref = 0;
-            return true;
-        }
-    }
-    else {
-        if(kTriEvery > 1 && iter % kTriEvery != 0u) return true; // taken in a later iteration
-        const int32_t leaf = ~T.ref;
-        if((uint32_t)leaf >= T.numFaces) {
-            trav_error(sc, kTravErrTriangle);
-            T.h.inst = kNoHit;
-            return false;
-        }
-        const u32x4* tp = reinterpret_cast<const u32x4*>(T.tris + leaf);
-        const u32x4 a = ld_global16(tp), b = ld_global16(tp + 1), cc = ld_global16(tp + 2);
+    else if(T.inBlas) { // a triangle
         Tri tri;
-        tri.v0x = __uint_as_float(a.x);
-        tri.v0y = __uint_as_float(a.y);
-        tri.v0z = __uint_as_float(a.z);
-        tri.prim = a.w;
-        tri.v1x = __uint_as_float(b.x);
-        tri.v1y = __uint_as_float(b.y);
-        tri.v1z = __uint_as_float(b.z);
-        tri.v2x = __uint_as_float(cc.x);
-        tri.v2y = __uint_as_float(cc.y);
-        tri.v2z = __uint_as_float(cc.z);
+        tri.v0x = __uint_as_float(v0.x);
+        tri.v0y = __uint_as_float(v0.y);
+        tri.v0z = __uint_as_float(v0.z);
+        tri.prim = v0.w;
+        tri.v1x = __uint_as_float(v1.x);
+        tri.v1y = __uint_as_float(v1.y);
+        tri.v1z = __uint_as_float(v1.z);
+        tri.v2x = __uint_as_float(v2.x);
+        tri.v2y = __uint_as_float(v2.y);
+        tri.v2z = __uint_as_float(v2.z);
         float t, u, v;
         if(wt_intersect(T.wt, tri, T.ray.tmin, T.tbest, t, u, v)) {
             T.tbest = t;
@@ -437,35 +398,66 @@ __device__ __forceinline__ bool trav_step(Traversal& T, const TraceScene& sc, St
             T.h.prim = tri.prim;
         }
     }
-    if(stack.sp == 0) return false;
-    T.ref = stack.pop();
+    else { // an instance: v3 = blas, mask, position, customIndex
+        if(v3.x >= sc.numBlas) {
+            trav_error(sc, kTravErrBlas);
+            T.h.inst = kNoHit;
+            return false;
+        }
+        const u32x4* bp = reinterpret_cast<const u32x4*>(sc.blas + v3.x);
+        const u32x4 b0 = ld_global16(bp);     // nodes, tris
+        const uint32_t numFaces = ld_global8(bp + 1).x;
+        if((v3.y & T.cullMask) != 0u && numFaces > 0u) {
+            const float w[12] = {__uint_as_float(v0.x), __uint_as_float(v0.y), __uint_as_float(v0.z), __uint_as_float(v0.w),
+                                 __uint_as_float(v1.x), __uint_as_float(v1.y), __uint_as_float(v1.z), __uint_as_float(v1.w),
+                                 __uint_as_float(v2.x), __uint_as_float(v2.y), __uint_as_float(v2.z), __uint_as_float(v2.w)};
+            float rox, roy, roz, rdx, rdy, rdz;
+            xform_ray(w, T.ray.ox, T.ray.oy, T.ray.oz, T.ray.dx, T.ray.dy, T.ray.dz, rox, roy, roz, rdx, rdy, rdz);
+            stack.set_box_ray(rox, roy, roz, safe_rcp(rdx), safe_rcp(rdy), safe_rcp(rdz));
+            const int rot = wt_setup(T.wt, rox, roy, roz, rdx, rdy, rdz);
+            stack.push(kSentinel);
+            T.nodes = reinterpret_cast<const char*>((uint64_t)b0.x | ((uint64_t)b0.y << 32));
+            // the copy of the triangles in this ray's axis order
+            T.leaves = reinterpret_cast<const char*>((uint64_t)b0.z | ((uint64_t)b0.w << 32)) + (uint64_t)rot * numFaces * sizeof(Tri);
+            T.leafStride = sizeof(Tri);
+            T.inBlas = true;
+            T.curInst = v3.z;
+            T.leafCap = numFaces;
+            T.nodeCap = numFaces > 2u ? numFaces - 1u : 1u;
+            T.ref = 0;
+            pop = false;
+        }
+    }
+    if(pop) {
+        if(stack.sp == 0) return false;
+        T.ref = stack.pop();
+        if(T.ref == kSentinel) { // back to the TLAS and its next entry (never a sentinel)
+            if(stack.sp == 0) return false;
+            T.ref = stack.pop();
+            enter_tlas(T, sc);
+            stack.set_box_ray(T.ray.ox, T.ray.oy, T.ray.oz, T.wix, T.wiy, T.wiz);
+        }
+    }
     return true;
 }
 
-// Iterations between a wave's instance entries / triangle tests / returns
-// to the TLAS (trav_step): the schedule of the traversal kernels, whose
-// lanes start their rays together (the queue pass, the ray queries and
-// each round of the drain).
+// Iterations between a wave's instance entries (trav_step): the schedule of
+// the traversal kernels, whose lanes start their rays together (the queue
+// pass, the ray queries and each round of the drain).
 #ifndef RGRT_INST_EVERY
-#define RGRT_INST_EVERY 4
-#endif
-#ifndef RGRT_TRI_EVERY
-#define RGRT_TRI_EVERY 1
-#endif
-#ifndef RGRT_SENT_EVERY
-#define RGRT_SENT_EVERY 1
+#define RGRT_INST_EVERY 2
 #endif
 
 // Whole traversal of one ray. Each node and leaf is visited at most once
 // per level, so a well-formed two-level tree ends far below the step cap;
 // the cap only bounds the loop.
-template<int kInstEvery = 1, int kTriEvery = 1, int kSentEvery = 1, typename Stack>
+template<int kInstEvery = 1, typename Stack>
 __device__ HitRec traverse(const TraceScene& sc, const RayIn& ray, uint32_t cullMask, Stack& stack)
 {
     Traversal T;
     if(trav_begin(T, sc, ray, cullMask, stack)) {
         for(uint32_t guard = 0; guard < (1u << 26); ++guard)
-            if(!trav_step<kInstEvery, kTriEvery, kSentEvery>(T, sc, stack, guard)) break;
+            if(!trav_step<kInstEvery>(T, sc, stack, guard)) break;
     }
     T.h.t = T.h.inst != kNoHit ? T.tbest : 0.0f;
     return T.h;

@@ -1107,7 +1107,7 @@ __device__ __forceinline__ void drain_scene(const ShadeParams& p, const TraceSce
         if(active) {
             // the active lanes start this traversal together, so the
             // wave-wide step schedule applies
-            const HitRec h = traverse<RGRT_INST_EVERY, RGRT_TRI_EVERY, RGRT_SENT_EVERY>(sc, r, (flags >> kMaskShift) & 0xffu, stack);
+            const HitRec h = traverse<RGRT_INST_EVERY>(sc, r, (flags >> kMaskShift) & 0xffu, stack);
             ++traced;
             OutRay out;
             if(advance_pixel<kNextSample>(c, pix, flags, f3(r.ox, r.oy, r.oz), f3(r.dx, r.dy, r.dz), h, P, sp, sample, out)) {
