@@ -13,7 +13,7 @@ namespace rgrt {
 uint32_t trace_spill_words_per_thread();
 uint32_t trace_block_size();
 void launch_trace_queue_impl(hipStream_t s, const TraceScene& sc, const WavefrontState& st, int cur, uint32_t gridBlocks,
-                             int32_t* spill, uint32_t* hostSlot);
+                             int32_t* spill, uint32_t* hostSlot, bool ahead);
 void launch_trace_rays_impl(hipStream_t s, const TraceScene& sc, const rgrt_ray* rays, uint32_t n, uint32_t cullMask,
                             rgrt_hit* hits, const InstanceShade* inst, int32_t* spill, uint32_t gridBlocks);
 } // namespace rgrt
@@ -394,6 +394,7 @@ void free_images(rgrt_ctx* c)
     dev_free(s.rays[0]);
     dev_free(s.rays[1]);
     dev_free(s.hits);
+    dev_free(s.ahead);
     dev_free(s.sampleAcc);
     dev_free(s.sampleLum2);
     c->slotCap = 0;
@@ -401,6 +402,26 @@ void free_images(rgrt_ctx* c)
     dev_free(s.counters);
     s.npix = 0;
 }
+
+// Whether a frame's shading passes queue reflection and refraction rays ahead
+// (wavefront.hip): it makes the chain of passes a third shorter, but the
+// shading kernel that takes such hits needs 155 VGPRs instead of 128. Small
+// frames wait on the chain; large ones, and several frames in flight, on the
+// work. Measured (pipelined): 640x360 0.587 -> 0.479 ms and with a rebuilt
+// mesh 0.635 -> 0.500, batches of 320x180 to 960x540 scenes 3.81 -> 3.39;
+// 960x540 over 3,000 instances 3.66 -> 3.89 and 1080p over 2M triangles 8.75
+// -> 9.8 ms. Slots that run several samples one after another keep the plain
+// kernels.
+constexpr uint32_t kAheadSlots = 300000;
+static_assert(kAheadSlots <= kAheadMaxSlots, "a queue entry names its slot");
+
+// Words of the suspended frames and of the queue of rays ahead for up to n
+// slots: a frame with fewer slots may be one with rays ahead.
+size_t frame_words(size_t n)
+{
+    return std::max(n * kFrameStride, std::min<size_t>(n, kAheadSlots) * kFrameStrideAhead) * kMaxFrames;
+}
+size_t ahead_words(size_t n) { return std::min<size_t>(n, kAheadSlots) * kAheadPerSlot * kAheadWords; }
 
 void alloc_images(rgrt_ctx* c, uint32_t w, uint32_t h)
 {
@@ -437,10 +458,11 @@ void alloc_images(rgrt_ctx* c, uint32_t w, uint32_t h)
     dev_alloc(s.payload, npix * kPayloadWords);
     dev_alloc(s.accum, npix * kAccumWords);
     dev_alloc(s.lum2, npix);
-    dev_alloc(s.frames, npix * kFrameStride * kMaxFrames);
+    dev_alloc(s.frames, frame_words(npix));
     dev_alloc(s.rays[0], npix * kRayWords);
     dev_alloc(s.rays[1], npix * kRayWords);
     dev_alloc(s.hits, npix * kHitWords);
+    dev_alloc(s.ahead, ahead_words(npix));
     dev_alloc(s.counters, 64);
     check(hipMemsetAsync(s.counters, 0, 64 * 4, c->stream));
     c->w = w;
@@ -521,6 +543,12 @@ void make_event(hipEvent_t& e)
 static_assert(sizeof(rgrt_stats) == 80, "rgrt_stats layout (Python binding: records.STATS_FIELDS)");
 static_assert(sizeof(rgrt_tuning) == 24, "rgrt_tuning layout (Python binding: records.TUNING)");
 
+// The frame in c->ubo (sample groups prepared) queues rays ahead.
+bool rays_ahead(const rgrt_ctx* c)
+{
+    return c->st.npix <= kAheadSlots && c->st.groups >= (uint32_t)std::max(1, c->ubo.numSamples);
+}
+
 ShadeParams shade_params(const rgrt_ctx* c)
 {
     ShadeParams p;
@@ -542,6 +570,7 @@ ShadeParams shade_params(const rgrt_ctx* c)
     p.keepAov = (c->flags & RGRT_CFG_PRIMARY_AOV) ? 1 : 0;
     p.sampling = c->sampling.mode;
     p.seed = c->sampling.seed;
+    p.aheadOn = rays_ahead(c) ? 1 : 0;
     return p;
 }
 
@@ -567,10 +596,11 @@ void prepare_sample_groups(rgrt_ctx* c)
     if(slots > c->slotCap) {
         check(hipStreamSynchronize(c->stream)); // queued frames still use the old arrays
         dev_alloc(s.payload, slots * kPayloadWords);
-        dev_alloc(s.frames, slots * kFrameStride * kMaxFrames);
+        dev_alloc(s.frames, frame_words(slots));
         dev_alloc(s.rays[0], slots * kRayWords);
         dev_alloc(s.rays[1], slots * kRayWords);
         dev_alloc(s.hits, slots * kHitWords);
+        dev_alloc(s.ahead, ahead_words(slots));
         c->slotCap = slots;
     }
     if(g > 1 && (size_t)n * s.nimg > c->sampleCap) {
@@ -684,13 +714,13 @@ rgrt_status do_trace(rgrt_ctx* c)
             }
             check(hipEventRecord(c->traceEvents[2 * traceLaunches], s));
         }
-        launch_trace_queue_impl(s, sc, c->st, cur, c->traceGrid, c->spill, c->hostCountsDev + it);
+        launch_trace_queue_impl(s, sc, c->st, cur, c->traceGrid, c->spill, c->hostCountsDev + it, p.aheadOn);
         check(hipEventRecord(c->iterEvents[it % ring], s));
         if(timing) {
             check(hipEventRecord(c->traceEvents[2 * traceLaunches + 1], s));
             check(hipEventRecord(c->shadeEvents[2 * traceLaunches], s));
         }
-        launch_shade(s, p, cur, c->shadeGrid);
+        launch_shade(s, p, cur, c->shadeGrid, it + 1 != c->tuning.wavefrontPasses);
         if(timing) check(hipEventRecord(c->shadeEvents[2 * traceLaunches + 1], s));
         ++traceLaunches;
         cur ^= 1;
@@ -726,8 +756,8 @@ void enqueue_trace_fixed(rgrt_ctx* c)
     launch_raygen(s, p);
     int cur = 0;
     for(uint32_t it = 0; it < passes; ++it) {
-        launch_trace_queue_impl(s, sc, c->st, cur, c->traceGrid, c->spill, c->hostCountsDev + it);
-        launch_shade(s, p, cur, c->shadeGrid);
+        launch_trace_queue_impl(s, sc, c->st, cur, c->traceGrid, c->spill, c->hostCountsDev + it, p.aheadOn);
+        launch_shade(s, p, cur, c->shadeGrid, it + 1 < passes);
         cur ^= 1;
     }
     launch_drain(s, p, sc, cur, c->drainGrid, c->spill);
@@ -768,6 +798,7 @@ WavefrontState band_state(const WavefrontState& st, uint32_t b, uint32_t bands)
     w.rays[0] = st.rays[0] + (size_t)kRayWords * q0;
     w.rays[1] = st.rays[1] + (size_t)kRayWords * q0;
     w.hits = st.hits + (size_t)kHitWords * q0;
+    w.ahead = st.ahead + (size_t)kAheadWords * kAheadPerSlot * q0;
     w.counters = st.counters + (size_t)kCounterBlock * b;
     return w;
 }
@@ -799,8 +830,8 @@ void enqueue_band(rgrt_ctx* c, uint32_t b, uint32_t bands, hipStream_t s)
     launch_raygen(s, p);
     int cur = 0;
     for(uint32_t it = 0; it < passes; ++it) {
-        launch_trace_queue_impl(s, sc, p.st, cur, c->traceGrid, spill, counts + it);
-        launch_shade(s, p, cur, c->shadeGrid);
+        launch_trace_queue_impl(s, sc, p.st, cur, c->traceGrid, spill, counts + it, p.aheadOn);
+        launch_shade(s, p, cur, c->shadeGrid, it + 1 < passes);
         cur ^= 1;
     }
     launch_drain(s, p, sc, cur, c->drainGrid, spill);

@@ -98,12 +98,23 @@ constexpr int kAccumWords = 12;
 // A suspended closest-hit frame: stage, material index, hit distance,
 // origin, direction, normal, the reference depth at the hit, shadow and
 // reflection colours and reflection depth (the material's values and the
-// grid effect are recomputed from these on resume), 19 words + 1 of padding.
-constexpr int kFrameStride = 20;
+// grid effect are recomputed from these on resume), 19 words + 1 of padding;
+// in a frame traced with rays ahead also the primitives those rays hit and the
+// index of refraction assumed for them (store_frame).
+constexpr int kFrameStride = 20, kFrameStrideAhead = 24;
 constexpr uint32_t kMaxMaterials = 1u << 28; // the material index shares a frame word with the stage
 constexpr int kMaxFrames = 8; // maxRecursions <= 7 keeps at most 7 frames waiting
 constexpr int kRayWords = 10; // origin, tmin, dir, tmax, pixel, flags
 constexpr int kHitWords = 5;
+// An entry of the queue of rays traced ahead (emit_ahead): origin, direction,
+// slot | level << 26 | kind << 29. A pass puts at most two per slot there.
+constexpr int kAheadWords = 7;
+constexpr int kAheadPerSlot = 2;
+constexpr uint32_t kAheadLevelShift = 26u, kAheadKindShift = 29u;
+constexpr uint32_t kAheadMaxSlots = 1u << kAheadLevelShift;
+constexpr uint32_t kAheadReflection = 0u, kAheadRefraction = 1u;
+constexpr float kAheadTmin = 0.01f, kAheadTmax = 1000.0f;
+constexpr int kAheadCountWord = 10; // in WavefrontState::counters: entries for the pass on queue 0, 1
 constexpr int kTraversalErrorWord = 12; // in WavefrontState::counters, sticky (cleared at allocation)
 constexpr int kCounterBlock = 16;       // counter words per band (the error word is band 0's)
 constexpr uint32_t kMaxBands = 4;
@@ -138,7 +149,8 @@ struct WavefrontState {
     float* frames = nullptr;  // [kMaxFrames][npix][kFrameStride]
     float* rays[2] = {nullptr, nullptr}; // [kRayWords][npix]
     float* hits = nullptr;    // [kHitWords][npix]
-    uint32_t* counters = nullptr; // [0..1] queue counts, [2..3] fetch, [4..11] stats (u64 pairs), [12] traversal errors
+    float* ahead = nullptr;   // [kAheadWords][kAheadPerSlot * npix]: rays traced ahead by the next pass
+    uint32_t* counters = nullptr; // [0..1] queue counts, [2..3] fetch, [4..9] stats (u64 pairs), [10..11] rays ahead, [12] traversal errors
     float* lum2 = nullptr;        // [npix]: sum of squared sample luminances (stochastic sampling)
 };
 
@@ -176,6 +188,7 @@ struct ShadeParams {
     int32_t keepAov;
     uint32_t sampling; // RGRT_SAMPLING_*
     uint32_t seed;
+    int32_t aheadOn; // shading passes may queue rays ahead (0: more slots than an entry can name)
 };
 
 // ---------------------------------------------------------------------------
@@ -287,7 +300,8 @@ void launch_drain_multi(hipStream_t s, const ShadeParams* ps, const TraceScene* 
 // start of a next sample.
 bool run_one_sample(const ShadeParams& p);
 void launch_trace_queue(hipStream_t s, const TraceScene& sc, const WavefrontState& st, int cur, uint32_t gridBlocks);
-void launch_shade(hipStream_t s, const ShadeParams& p, int cur, uint32_t gridBlocks);
+// ahead: a traversal pass follows this shading pass (not the drain)
+void launch_shade(hipStream_t s, const ShadeParams& p, int cur, uint32_t gridBlocks, bool ahead);
 void launch_finalize_samples(hipStream_t s, const ShadeParams& p);
 void launch_drain(hipStream_t s, const ShadeParams& p, const TraceScene& sc, int cur, uint32_t gridBlocks, int32_t* spill);
 uint32_t drain_spill_words_per_thread();

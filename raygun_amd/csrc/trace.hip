@@ -13,8 +13,9 @@ constexpr int kTraceBlock = 256;
 constexpr int kLdsStack = 16;
 constexpr int kSpill = 368; // with the 16 LDS entries: the 381-entry worst case of two wide LBVH levels
 
-// Wavefront trace pass: rays [0, count) of queue `cur` -> hit records.
-// Waves fetch 64 rays at a time from a global counter (persistent grid).
+// Wavefront trace pass: rays [0, count) of queue `cur` -> hit records, and
+// the rays queued ahead -> the frames that will need their hits. Waves fetch
+// 64 rays at a time from a global counter (persistent grid).
 // Waves per SIMD the traversal pass is compiled for: the register budget is
 // 512 / waves VGPRs. At 7 waves (73) nine registers spill in the loop: a
 // 1080p frame over 2M triangles takes 8.92 ms against 8.75 at 6 waves, 3,000
@@ -23,56 +24,88 @@ constexpr int kSpill = 368; // with the 16 LDS entries: the 381-entry worst case
 #define RGRT_TRACE_WAVES 6
 #endif
 
-__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(RGRT_TRACE_WAVES))) void k_trace_queue(TraceScene sc, const float* __restrict__ rays,
-                                                              float* __restrict__ hits, uint32_t npix,
-                                                              uint32_t* __restrict__ counters, int cur,
-                                                              int32_t* __restrict__ spillBase, uint32_t* hostSlot)
+template<bool kAhead>
+__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(RGRT_TRACE_WAVES))) void k_trace_queue(
+    TraceScene sc, WavefrontState st, int cur, int32_t* __restrict__ spillBase, uint32_t* hostSlot)
 {
     __shared__ int32_t ldsStack[kLdsStack * kTraceBlock];
+    uint32_t* counters = st.counters;
+    const float* __restrict__ rays = st.rays[cur];
+    float* __restrict__ hits = st.hits;
+    const size_t npix = st.npix;
+    const size_t aheadCap = npix * kAheadPerSlot;
     const uint32_t count = counters[cur];
+    const uint32_t ahead = kAhead ? (uint32_t)min((size_t)counters[kAheadCountWord + cur], aheadCap) : 0u;
     if(blockIdx.x == 0 && threadIdx.x == 0) {
-        *hostSlot = count;         // host-visible: lets the host stop once the queues drain
-        counters[1 - cur] = 0;     // the output queue of the shading pass that follows
+        *hostSlot = count + ahead; // host-visible: lets the host stop once the queues drain
+        counters[1 - cur] = 0;     // the output queues of the shading pass that follows
+        counters[kAheadCountWord + (1 - cur)] = 0;
         counters[2 + (1 - cur)] = 0; // the fetch counter of the next traversal pass
         // ray statistics (64-bit) at counters[4..5]
-        atomicAdd(reinterpret_cast<unsigned long long*>(counters + 4), (unsigned long long)count);
+        atomicAdd(reinterpret_cast<unsigned long long*>(counters + 4), (unsigned long long)count + ahead);
     }
     const int lane = threadIdx.x & 63;
     const uint32_t gtid = blockIdx.x * kTraceBlock + threadIdx.x;
     __shared__ float boxRay[kBoxRayWords * kTraceBlock];
     TraversalStack<kLdsStack, kTraceBlock, kSpill> stack{ldsStack, spillBase + (size_t)gtid * kSpill, (int)threadIdx.x, boxRay};
     uint32_t* fetch = counters + 2 + cur;
-    // Wave w first takes rays [64w, 64w + 64); rays beyond the grid's static
-    // share are fetched 64 at a time from a counter, so a pass with fewer
-    // rays than the grid has lanes does no atomics at all.
+    // The work is cut into chunks of 64 rays: the queue's, then those of the
+    // rays queued ahead. Wave w first takes chunk w; chunks beyond the grid's
+    // static share are fetched from a counter, so a pass with fewer rays than
+    // the grid has lanes does no atomics at all.
     const uint32_t wavesInGrid = gridDim.x * (kTraceBlock / 64);
-    const uint32_t dynStart = wavesInGrid * 64u;
-    uint32_t base = (blockIdx.x * (kTraceBlock / 64) + (threadIdx.x >> 6)) * 64u;
-    for(;;) {
-        if(base >= count) break;
-        const uint32_t i = base + lane;
-        if(i < count) {
+    const uint32_t mainChunks = (count + 63u) / 64u;
+    const uint32_t chunks = mainChunks + (ahead + 63u) / 64u;
+    uint32_t k = blockIdx.x * (kTraceBlock / 64) + (threadIdx.x >> 6);
+    while(k < chunks) {
+        const bool isAhead = kAhead && k >= mainChunks;
+        const uint32_t i = (isAhead ? k - mainChunks : k) * 64u + lane;
+        if(i < (isAhead ? ahead : count)) {
             RayIn r;
-            r.ox = rays[0 * (size_t)npix + i];
-            r.oy = rays[1 * (size_t)npix + i];
-            r.oz = rays[2 * (size_t)npix + i];
-            r.tmin = rays[3 * (size_t)npix + i];
-            r.dx = rays[4 * (size_t)npix + i];
-            r.dy = rays[5 * (size_t)npix + i];
-            r.dz = rays[6 * (size_t)npix + i];
-            r.tmax = rays[7 * (size_t)npix + i];
-            const uint32_t flags = __float_as_uint(rays[9 * (size_t)npix + i]);
-            const HitRec h = traverse<RGRT_INST_EVERY>(sc, r, (flags >> kMaskShift) & 0xffu, stack);
-            hits[0 * (size_t)npix + i] = h.t;
-            hits[1 * (size_t)npix + i] = h.u;
-            hits[2 * (size_t)npix + i] = h.v;
-            hits[3 * (size_t)npix + i] = __uint_as_float(h.inst);
-            hits[4 * (size_t)npix + i] = __uint_as_float(h.prim);
+            uint32_t mask, slot = 0;
+            if(isAhead) {
+                const float* q = st.ahead + i;
+                r.ox = q[0 * aheadCap];
+                r.oy = q[1 * aheadCap];
+                r.oz = q[2 * aheadCap];
+                r.dx = q[3 * aheadCap];
+                r.dy = q[4 * aheadCap];
+                r.dz = q[5 * aheadCap];
+                slot = __float_as_uint(q[6 * aheadCap]);
+                r.tmin = kAheadTmin;
+                r.tmax = kAheadTmax;
+                mask = 0xffu;
+            }
+            else {
+                r.ox = rays[0 * npix + i];
+                r.oy = rays[1 * npix + i];
+                r.oz = rays[2 * npix + i];
+                r.tmin = rays[3 * npix + i];
+                r.dx = rays[4 * npix + i];
+                r.dy = rays[5 * npix + i];
+                r.dz = rays[6 * npix + i];
+                r.tmax = rays[7 * npix + i];
+                mask = (__float_as_uint(rays[9 * npix + i]) >> kMaskShift) & 0xffu;
+            }
+            const HitRec h = traverse<RGRT_INST_EVERY>(sc, r, mask, stack);
+            if(isAhead) { // into the frame that waits for it (store_frame)
+                const uint32_t level = (slot >> kAheadLevelShift) & 7u, kind = slot >> kAheadKindShift;
+                float* b = st.frames + ((size_t)level * st.frameSlots + (slot & (kAheadMaxSlots - 1u))) * kFrameStrideAhead;
+                reinterpret_cast<float4*>(b)[3 + kind] = make_float4(h.t, h.u, h.v, __uint_as_float(h.inst));
+                b[20 + kind] = __uint_as_float(h.prim);
+            }
+            else {
+                hits[0 * npix + i] = h.t;
+                hits[1 * npix + i] = h.u;
+                hits[2 * npix + i] = h.v;
+                hits[3 * npix + i] = __uint_as_float(h.inst);
+                hits[4 * npix + i] = __uint_as_float(h.prim);
+            }
         }
-        if(count <= dynStart) break; // no rays beyond the static share
+        if(chunks <= wavesInGrid) break; // no rays beyond the static share
         uint32_t b = 0;
-        if(lane == 0) b = dynStart + atomicAdd(fetch, 64u);
-        base = __shfl(b, 0);
+        if(lane == 0) b = wavesInGrid + atomicAdd(fetch, 1u);
+        k = __shfl(b, 0);
     }
 }
 
@@ -192,9 +225,10 @@ uint32_t trace_spill_words_per_thread() { return kSpill; }
 uint32_t trace_block_size() { return kTraceBlock; }
 
 void launch_trace_queue_impl(hipStream_t s, const TraceScene& sc, const WavefrontState& st, int cur, uint32_t gridBlocks,
-                             int32_t* spill, uint32_t* hostSlot)
+                             int32_t* spill, uint32_t* hostSlot, bool ahead)
 {
-    k_trace_queue<<<gridBlocks, kTraceBlock, 0, s>>>(sc, st.rays[cur], st.hits, st.npix, st.counters, cur, spill, hostSlot);
+    if(ahead) k_trace_queue<true><<<gridBlocks, kTraceBlock, 0, s>>>(sc, st, cur, spill, hostSlot);
+    else k_trace_queue<false><<<gridBlocks, kTraceBlock, 0, s>>>(sc, st, cur, spill, hostSlot);
 }
 
 void launch_trace_multi(hipStream_t s, const ShadeParams* ps, const TraceScene* scs, int numScenes, int cur, uint32_t gridBlocks,

@@ -20,6 +20,15 @@
 //   SI_TRACE   shadow-internal, after SHADOW_TRACE  :133-138
 //   SI_SKY     shadow-internal, after the sky ray   :144-145
 //   ST_INTERNAL shadow-trace, after SHADOW_INTERNAL :158-159
+// A hit's reflection and refraction rays are known at the hit, before its
+// shadow ray's own chain has run, and a traversal depends on nothing but the
+// ray. A shading pass therefore queues them beside the ray the pixel waits
+// for, the next traversal pass traces all of them, and when the frame comes to
+// its reflection or refraction it finds that hit and shades on at once
+// instead of waiting for a pass of its own. Order and results are those of
+// one ray at a time; only the refraction's direction can turn out different
+// (its index of refraction is the payload's when its turn comes, and a
+// reflection before it may change that): such a ray is traced again.
 // A ray with cull mask 0 (:144) cannot hit and a refraction ray with a zero
 // direction (refract() at total internal reflection) is defined here not to
 // hit either; both go straight to their miss shader without a queue entry.
@@ -57,6 +66,13 @@ constexpr int kShadeBlock = 256;
 // frame with four frames in flight.
 #ifndef RGRT_DRAIN1_WAVES
 #define RGRT_DRAIN1_WAVES 4
+#endif
+
+#ifndef RGRT_SHADE_AHEAD_WAVES
+#define RGRT_SHADE_AHEAD_WAVES 3
+#endif
+#ifndef RGRT_DRAIN_AHEAD_WAVES
+#define RGRT_DRAIN_AHEAD_WAVES 3
 #endif
 
 enum Stage : int { G_SHADOW = 1, G_REFL = 2, G_REFR = 3, SI_TRACE = 4, SI_SKY = 5, ST_INTERNAL = 6 };
@@ -105,6 +121,7 @@ struct Frame {
     float emission;
     F3 baseColor, shadowColor, reflectColor;
     float reflectDepth;
+    uint32_t ahead; // bit kAheadReflection / kAheadRefraction: that ray was queued ahead
 };
 
 struct OutRay {
@@ -120,7 +137,8 @@ struct Ctx {
     const ShadeParams& p;
     F3 L;
     int maxRec;
-    uint32_t key; // sample key of the ray being shaded (stochastic sampling)
+    uint32_t key;    // sample key of the ray being shaded (stochastic sampling)
+    uint32_t* ahead; // count of the rays queued ahead for the next pass; null: none are
 };
 
 // ---------------------------------------------------------------------------
@@ -160,9 +178,16 @@ __device__ __forceinline__ void store_state(const ShadeParams& p, uint32_t pix, 
     b[1] = make_float4(P.curIOR, P.refDepth, __int_as_float(P.recDepth), __uint_as_float(m));
 }
 
-// Frame record (kFrameStride words) in five 16-byte parts: [0] stage |
+// Frame record (kFrameStride words, kFrameStrideAhead with rays ahead) in
+// 16-byte parts: [0] stage |
 // frontFacing << 3 | mat << 4, t, origin.xy; [1] origin.z, dir; [2] vn,
-// gridRef; [3] shadowColor, reflectDepth; [4] reflectColor, 0.
+// gridRef; [3] shadowColor, reflectDepth; [4] reflectColor, 0; [5] see below.
+// A ray queued ahead sets the sign of t (reflection) or gridRef (refraction),
+// both distances >= 0. The traversal puts the reflection's t, u, v, instance
+// in [3] and primitive in [5].x, the refraction's in [4] and [5].y; [5].z is
+// the index of refraction the refraction ray assumed. No stage reads [3] or
+// [4] before the hit there has been taken (take_ahead): a frame in G_SHADOW
+// uses neither, one in G_REFL not [4].
 // Only the parts a later resume reads and that changed are written: a frame
 // suspended by the closest-hit stage (`fresh`) writes [0..2]; [3] once a
 // stage after it reads shadowColor or reflectDepth (every stage but G_SHADOW,
@@ -170,18 +195,64 @@ __device__ __forceinline__ void store_state(const ShadeParams& p, uint32_t pix, 
 // them, and ST_INTERNAL, which reads nothing but the stage); [4] for G_REFR,
 // the only stage whose resume reads reflectColor. A resumed frame's [1], [2]
 // are unchanged in memory.
+template<bool kAhead>
+__device__ __forceinline__ float* frame_record(const ShadeParams& p, uint32_t pix, int level)
+{
+    return p.st.frames + ((size_t)level * p.st.frameSlots + pix) * (kAhead ? kFrameStrideAhead : kFrameStride);
+}
+
+template<bool kAhead>
 __device__ __forceinline__ void store_frame(const ShadeParams& p, uint32_t pix, int level, const Frame& F, bool fresh)
 {
-    float4* b = reinterpret_cast<float4*>(p.st.frames + ((size_t)level * p.st.frameSlots + pix) * kFrameStride);
+    float4* b = reinterpret_cast<float4*>(frame_record<kAhead>(p, pix, level));
     const uint32_t w0 = ((uint32_t)F.stage & 7u) | (((uint32_t)F.frontFacing & 1u) << 3) | (F.mat << 4);
-    b[0] = make_float4(__uint_as_float(w0), F.t, F.origin.x, F.origin.y);
+    b[0] = make_float4(__uint_as_float(w0), kAhead && ((F.ahead >> kAheadReflection) & 1u) ? -F.t : F.t, F.origin.x, F.origin.y);
     if(fresh) {
         b[1] = make_float4(F.origin.z, F.dir.x, F.dir.y, F.dir.z);
-        b[2] = make_float4(F.vn.x, F.vn.y, F.vn.z, F.gridRef);
+        b[2] = make_float4(F.vn.x, F.vn.y, F.vn.z, kAhead && ((F.ahead >> kAheadRefraction) & 1u) ? -F.gridRef : F.gridRef);
     }
     if(F.stage != G_SHADOW && F.stage != ST_INTERNAL)
         b[3] = make_float4(F.shadowColor.x, F.shadowColor.y, F.shadowColor.z, F.reflectDepth);
     if(F.stage == G_REFR) b[4] = make_float4(F.reflectColor.x, F.reflectColor.y, F.reflectColor.z, 0.0f);
+}
+
+// Queues a ray of the frame being suspended at `level` for the next traversal
+// pass. Any subset of a wave's lanes may call it: one atomic for the lanes that
+// are here.
+__device__ __forceinline__ void emit_ahead(const ShadeParams& p, uint32_t* count, uint32_t pix, int level, uint32_t kind, F3 o, F3 d)
+{
+    const uint64_t here = __ballot(1);
+    const int lane = (int)__lane_id();
+    const int first = __ffsll((unsigned long long)here) - 1;
+    uint32_t base = 0;
+    if(lane == first) base = atomicAdd(count, (uint32_t)__popcll(here));
+    base = (uint32_t)__builtin_amdgcn_readlane((int)base, first);
+    const uint32_t i = base + (uint32_t)__popcll(here & (lane == 0 ? 0ull : ((~0ull) >> (64 - lane))));
+    const size_t n = (size_t)p.st.npix * kAheadPerSlot;
+    if(i >= n) return; // cannot happen: two per slot and pass
+    float* q = p.st.ahead + i;
+    q[0 * n] = o.x;
+    q[1 * n] = o.y;
+    q[2 * n] = o.z;
+    q[3 * n] = d.x;
+    q[4 * n] = d.y;
+    q[5 * n] = d.z;
+    q[6 * n] = __uint_as_float(pix | ((uint32_t)level << kAheadLevelShift) | (kind << kAheadKindShift));
+}
+
+// The hit of a ray queued ahead by the frame at `level` (before store_frame
+// writes the frame's next stage over it).
+__device__ __forceinline__ HitRec take_ahead(const ShadeParams& p, uint32_t pix, int level, uint32_t kind)
+{
+    const float* b = frame_record<true>(p, pix, level);
+    const float4 a = reinterpret_cast<const float4*>(b)[3 + kind];
+    HitRec h;
+    h.t = a.x;
+    h.u = a.y;
+    h.v = a.z;
+    h.inst = __float_as_uint(a.w);
+    h.prim = __float_as_uint(b[20 + kind]);
+    return h;
 }
 
 __device__ __forceinline__ void init_payload(Payload& P) // raygen.h:92-100
@@ -317,24 +388,57 @@ __device__ void generic_finish(const Frame& F, Payload& P, F3 refractColor)
     P.depth = F.t;
 }
 
-// Refraction part (closesthit.rchit:223-251).
-__device__ int generic_refraction(const Ctx& c, Frame& F, Payload& P, OutRay& out)
+// Direction of the refraction ray (closesthit.rchit:225-231, 238-243) of a
+// payload with index of refraction curIOR.
+__device__ __forceinline__ F3 refraction_dir(const Frame& F, float curIOR)
+{
+    if(F.frontFacing) return refract(F.dir, F.vn, curIOR / F.ior);
+    return refract(F.dir, F.vn, F.ior / 1.0f);
+}
+
+// Direction of the reflection ray (closesthit.rchit:212-213).
+__device__ __forceinline__ F3 reflection_dir(const Ctx& c, const Frame& F)
+{
+    F3 dir = reflect(F.dir, F.vn);
+    if(c.p.sampling == RGRT_SAMPLING_STOCHASTIC && F.roughness > 0.0f)
+        dir = glossy_dir(c.key, F.origin, dir, F.vn, F.roughness);
+    return dir;
+}
+
+// Queues the rays a fresh frame (to be stored at `level`) will need after the
+// one it issues now.
+__device__ __forceinline__ void rays_ahead(const Ctx& c, Frame& F, const Payload& P, uint32_t pix, int level, bool reflection)
+{
+    if(!c.ahead || level >= kMaxFrames) return;
+    if(reflection && F.reflectivity > 0.0f) {
+        emit_ahead(c.p, c.ahead, pix, level, kAheadReflection, F.origin, reflection_dir(c, F));
+        F.ahead |= 1u << kAheadReflection;
+    }
+    if(F.transparency > 0.0f) {
+        const F3 d = refraction_dir(F, P.curIOR);
+        if(d.x != 0.0f || d.y != 0.0f || d.z != 0.0f) { // total internal reflection traces no ray
+            emit_ahead(c.p, c.ahead, pix, level, kAheadRefraction, F.origin, d);
+            F.ahead |= 1u << kAheadRefraction;
+            frame_record<true>(c.p, pix, level)[22] = P.curIOR;
+        }
+    }
+}
+
+// Refraction part (closesthit.rchit:223-251). `level`: the frame's.
+template<bool kAhead>
+__device__ int generic_refraction(const Ctx& c, Frame& F, Payload& P, OutRay& out, uint32_t pix, int level)
 {
     if(P.recDepth < c.maxRec && F.transparency > 0.0f) {
-        F3 dir;
-        if(F.frontFacing) {
-            const float eta = P.curIOR / F.ior;
-            dir = refract(F.dir, F.vn, eta);
-            P.recDepth++;
-            P.curIOR = F.ior;
+        if(kAhead && ((F.ahead >> kAheadRefraction) & 1u) && F.frontFacing &&
+           frame_record<true>(c.p, pix, level)[22] != P.curIOR) {
+            // assumed another index of refraction: that ray was not this one
+            F.ahead &= ~(1u << kAheadRefraction);
+            atomicAdd(reinterpret_cast<unsigned long long*>(c.p.st.counters + 4), ~0ull);
         }
-        else {
-            const float eta = F.ior / 1.0f;
-            dir = refract(F.dir, F.vn, eta);
-            P.recDepth++;
-            P.curIOR = 1.0f;
-        }
-        set_ray(out, F.origin, 0.01f, dir, 1000.0f, 0xffu, 0u);
+        const F3 dir = refraction_dir(F, P.curIOR);
+        P.recDepth++;
+        P.curIOR = F.frontFacing ? F.ior : 1.0f;
+        set_ray(out, F.origin, kAheadTmin, dir, kAheadTmax, 0xffu, 0u);
         F.stage = G_REFR;
         return EMIT_FRAME;
     }
@@ -342,22 +446,23 @@ __device__ int generic_refraction(const Ctx& c, Frame& F, Payload& P, OutRay& ou
     return RET;
 }
 
-// Reflection part (closesthit.rchit:206-221).
-__device__ int generic_reflection(const Ctx& c, Frame& F, Payload& P, OutRay& out)
+// Reflection part (closesthit.rchit:206-221). `fresh`: called by the hit
+// itself (it issued no shadow ray).
+template<bool kAhead>
+__device__ int generic_reflection(const Ctx& c, Frame& F, Payload& P, OutRay& out, uint32_t pix, int level, bool fresh)
 {
     F.reflectColor = f3(1.0f);
     F.reflectDepth = 0.0f;
     if(P.recDepth < c.maxRec && F.reflectivity > 0.0f) {
-        F3 dir = reflect(F.dir, F.vn);
-        if(c.p.sampling == RGRT_SAMPLING_STOCHASTIC && F.roughness > 0.0f)
-            dir = glossy_dir(c.key, F.origin, dir, F.vn, F.roughness);
+        if(kAhead && fresh) rays_ahead(c, F, P, pix, level, false);
+        const F3 dir = reflection_dir(c, F);
         P.recDepth += F.rayConsumption;
         P.refDepth += F.t;
-        set_ray(out, F.origin, 0.01f, dir, 1000.0f, 0xffu, 0u);
+        set_ray(out, F.origin, kAheadTmin, dir, kAheadTmax, 0xffu, 0u);
         F.stage = G_REFL;
         return EMIT_FRAME;
     }
-    return generic_refraction(c, F, P, out);
+    return generic_refraction<kAhead>(c, F, P, out, pix, level);
 }
 
 __device__ void grid_effect(float refDepth, float hitT, Frame& F, F3 pos) // closesthit.rchit:74-91
@@ -399,10 +504,11 @@ __device__ __forceinline__ void frame_material(const ShadeParams& p, Frame& F)
 // closest-hit stage had derived from them (material, grid effect and
 // baseColor = max(dot(-L, vn), 0.2) * diffuse, closesthit.rchit:174-175),
 // with the same operations on the same values.
+template<bool kAhead>
 __device__ __forceinline__ void load_frame(const Ctx& c, uint32_t pix, int level, Frame& F)
 {
     const ShadeParams& p = c.p;
-    const float4* b = reinterpret_cast<const float4*>(p.st.frames + ((size_t)level * p.st.frameSlots + pix) * kFrameStride);
+    const float4* b = reinterpret_cast<const float4*>(frame_record<kAhead>(p, pix, level));
     // all five parts in one go (reading only the written ones would wait for
     // the stage first); parts store_frame skipped hold values that are set
     // before they are read
@@ -411,11 +517,12 @@ __device__ __forceinline__ void load_frame(const Ctx& c, uint32_t pix, int level
     F.stage = (int)(w0 & 7u);
     F.frontFacing = (int)((w0 >> 3) & 1u);
     F.mat = min(w0 >> 4, p.numMaterials ? p.numMaterials - 1 : 0u); // as stored; the clamp only guards the table
-    F.t = a0.y;
+    F.ahead = kAhead ? (__float_as_uint(a0.y) >> 31) << kAheadReflection | (__float_as_uint(a2.w) >> 31) << kAheadRefraction : 0u;
+    F.t = kAhead ? fabsf(a0.y) : a0.y;
     F.origin = f3(a0.z, a0.w, a1.x);
     F.dir = f3(a1.y, a1.z, a1.w);
     F.vn = f3(a2.x, a2.y, a2.z);
-    F.gridRef = a2.w;
+    F.gridRef = kAhead ? fabsf(a2.w) : a2.w;
     F.shadowColor = f3(a3.x, a3.y, a3.z);
     F.reflectDepth = a3.w;
     F.reflectColor = f3(a4.x, a4.y, a4.z);
@@ -464,10 +571,12 @@ __device__ const rgrt_material& hit_material(const ShadeParams& p, uint32_t inst
     return p.mats[p.numMaterials ? min(mi, p.numMaterials - 1) : 0u];
 }
 
+template<bool kAhead>
 __device__ int closest_hit(const Ctx& c, Payload& P, uint32_t instPos, uint32_t prim, float hitT, float u, float v, F3 O, F3 D,
-                           Frame& F, OutRay& out)
+                           Frame& F, OutRay& out, uint32_t pix, int level)
 {
     const ShadeParams& p = c.p;
+    F.ahead = 0u;
     // Gathers are clamped to the buffers: an inconsistent offset table reads
     // wrong data (as the reference would) but never outside an allocation.
     const InstanceShade& is = p.inst[min(instPos, p.numInstances - 1)];
@@ -556,6 +665,7 @@ __device__ int closest_hit(const Ctx& c, Payload& P, uint32_t instPos, uint32_t 
         if(P.recDepth < c.maxRec) {
             P.hitValue = f3(1.0f);
             P.rayType = RT_SHADOW_TRACE;
+            if(kAhead) rays_ahead(c, F, P, pix, level, true);
             P.recDepth++;
             set_ray(out, origin, tmin * 10.0f, -c.L, tmax, 0xffu, 1u);
             F.stage = G_SHADOW;
@@ -566,23 +676,24 @@ __device__ int closest_hit(const Ctx& c, Payload& P, uint32_t instPos, uint32_t 
         const float shadowModulation = powf(F.transparency, 2.0f);
         F.shadowColor = F.transparency < 1.0f ? mix(f3(1.0f), F.diffuse * shadowModulation, F.transparency) : f3(0.4f);
     }
-    return generic_reflection(c, F, P, out);
+    return generic_reflection<kAhead>(c, F, P, out, pix, level, true);
 }
 
 // Continuation of a suspended frame once its nested trace returned.
-__device__ int resume(const Ctx& c, Frame& F, Payload& P, OutRay& out)
+template<bool kAhead>
+__device__ int resume(const Ctx& c, Frame& F, Payload& P, OutRay& out, uint32_t pix, int level)
 {
     switch(F.stage) {
     case G_SHADOW:
         P.recDepth--;
         F.shadowColor = P.hitValue;
         P.rayType = RT_GENERIC;
-        return generic_reflection(c, F, P, out);
+        return generic_reflection<kAhead>(c, F, P, out, pix, level, false);
     case G_REFL:
         P.recDepth -= F.rayConsumption;
         F.reflectColor = P.hitValue * F.specular;
         F.reflectDepth = P.depth;
-        return generic_refraction(c, F, P, out);
+        return generic_refraction<kAhead>(c, F, P, out, pix, level);
     case G_REFR: {
         P.recDepth--;
         F3 refractColor;
@@ -765,7 +876,7 @@ __device__ __forceinline__ void raygen_slot(const ShadeParams& p, uint32_t q)
         c[1] = 0;
         c[2] = 0;
         c[3] = 0;
-        for(int k = 4; k < 12; ++k) c[k] = 0; // ray / sky / zero-dir counters (u64)
+        for(int k = 4; k < 12; ++k) c[k] = 0; // ray / sky / zero-dir counters (u64), rays ahead
     }
     if(q >= p.st.npix) return;
     const uint32_t pix = p.st.chunkFirst * 64u + q;
@@ -844,12 +955,14 @@ __global__ __launch_bounds__(kShadeBlock) void k_finalize_samples(ShadeParams p)
 // slot's next sample (its camera ray needs the frame's two matrices, ~22
 // VGPRs at the kernels' peak): valid when every slot runs one sample, i.e.
 // sample groups >= samples (the launchers pick; see run_one_sample).
-template<bool kNextSample>
-__device__ bool advance_pixel(const Ctx& c0, uint32_t pix, uint32_t flags, F3 O, F3 D, const HitRec& h, Payload& P, int& sp,
-                              int& sample, OutRay& out)
+// kAhead compiles in the taking of rays traced ahead (and their queueing where
+// c.ahead is set).
+template<bool kNextSample, bool kAhead>
+__device__ bool advance_pixel(const Ctx& c0, uint32_t pix, uint32_t flags, F3 O, F3 D, HitRec h, Payload& P, int& sp, int& sample,
+                              OutRay& out)
 {
     const ShadeParams& p = c0.p;
-    Ctx c{c0.p, c0.L, c0.maxRec, 0u};
+    Ctx c{c0.p, c0.L, c0.maxRec, 0u, c0.ahead};
     const uint32_t tile = slot_image(p, pix); // the pixel in tile order
     uint32_t imgPix = 0;
     if(p.sampling == RGRT_SAMPLING_STOCHASTIC) {
@@ -883,60 +996,82 @@ __device__ bool advance_pixel(const Ctx& c0, uint32_t pix, uint32_t flags, F3 O,
         slot_pixel(tile, p.width, p.height, px, py);
         p.img.primary[py * p.width + px] = a;
     }
-    Frame F;
-    int step;
-    bool fresh = true; // F comes from the closest-hit stage, not from a resume
-    if(h.inst != kNoHit) {
-        step = closest_hit(c, P, h.inst, h.prim, h.t, h.u, h.v, O, D, F, out);
-    }
-    else {
-        run_miss(c, P, D, flags & kFlagMiss1);
-        step = RET;
-    }
-    for(;;) {
-        if(step == EMIT_FRAME) {
-            if(sp < kMaxFrames) store_frame(p, pix, sp, F, fresh);
-            sp++;
-            step = EMIT;
+    uint32_t miss1 = flags & kFlagMiss1;
+    for(;;) { // a hit (or miss) and what it returns into
+        Frame F;
+        int step;
+        if(kAhead) asm volatile("" : "+v"(pix)); // keeps the loop's addresses out of registers across it
+        bool fresh = true; // F comes from the closest-hit stage, not from a resume
+        if(h.inst != kNoHit) {
+            step = closest_hit<kAhead>(c, P, h.inst, h.prim, h.t, h.u, h.v, O, D, F, out, pix, sp);
         }
-        if(step == EMIT) {
-            if(out.mask == 0u) {
-                atomicAdd(skyCount, 1ull);
-                run_miss(c, P, out.d, out.miss1);
-                step = RET;
-            }
-            else if(out.d.x == 0.0f && out.d.y == 0.0f && out.d.z == 0.0f) {
-                atomicAdd(zeroCount, 1ull);
-                run_miss(c, P, out.d, out.miss1);
-                step = RET;
-            }
-            else {
-                return true;
-            }
+        else {
+            run_miss(c, P, D, miss1);
+            step = RET;
         }
-        // step == RET: the innermost call returned
-        if(sp == 0) {
-            if(p.st.groups == 1u)
-                accumulate(p, pix, P);
-            else
-                store_sample(p, tile, sample, P);
-            sample += (int)p.st.groups;
-            if(kNextSample && sample < p.ubo.numSamples) {
-                init_payload(P);
-                uint32_t px, py;
-                slot_pixel(tile, p.width, p.height, px, py);
-                primary_ray(p.ubo, px, py, p.width, p.height, sample, p.sampling, p.seed, out);
-                if(p.sampling == RGRT_SAMPLING_STOCHASTIC) c.key = sample_key(p.seed, imgPix, (uint32_t)sample);
+        for(;;) {
+            if(step == EMIT_FRAME) {
+                // the ray may have been traced ahead (only a resumed frame's)
+                const uint32_t kind = F.stage == G_REFR ? kAheadRefraction : kAheadReflection;
+                const bool taken = kAhead && !fresh && (F.stage == G_REFL || F.stage == G_REFR) && ((F.ahead >> kind) & 1u);
+                if(taken) {
+                    h = take_ahead(p, pix, sp, kind);
+                    O = out.o;
+                    D = out.d;
+                    miss1 = 0u;
+                }
+                if(sp < kMaxFrames) store_frame<kAhead>(p, pix, sp, F, fresh);
+                sp++;
+                if(taken) {
+                    // as in a pass of its own (load_state): the outermost hit
+                    // writes these last
+                    P.normal = f3(0.0f);
+                    P.rv[0] = P.rv[1] = P.rv[2] = P.rv[3] = 0.0f;
+                    P.reflectContribution = 0.0f;
+                    break;
+                }
                 step = EMIT;
-                continue;
             }
-            if(p.st.groups == 1u) finalize(p, pix); // otherwise k_finalize_samples does
-            return false;
+            if(step == EMIT) {
+                if(out.mask == 0u) {
+                    atomicAdd(skyCount, 1ull);
+                    run_miss(c, P, out.d, out.miss1);
+                    step = RET;
+                }
+                else if(out.d.x == 0.0f && out.d.y == 0.0f && out.d.z == 0.0f) {
+                    atomicAdd(zeroCount, 1ull);
+                    run_miss(c, P, out.d, out.miss1);
+                    step = RET;
+                }
+                else {
+                    return true;
+                }
+            }
+            // step == RET: the innermost call returned
+            if(sp == 0) {
+                if(p.st.groups == 1u)
+                    accumulate(p, pix, P);
+                else
+                    store_sample(p, tile, sample, P);
+                sample += (int)p.st.groups;
+                if(kNextSample && sample < p.ubo.numSamples) {
+                    init_payload(P);
+                    uint32_t px, py;
+                    slot_pixel(tile, p.width, p.height, px, py);
+                    primary_ray(p.ubo, px, py, p.width, p.height, sample, p.sampling, p.seed, out);
+                    if(p.sampling == RGRT_SAMPLING_STOCHASTIC) c.key = sample_key(p.seed, imgPix, (uint32_t)sample);
+                    step = EMIT;
+                    continue;
+                }
+                if(p.st.groups == 1u) finalize(p, pix); // otherwise k_finalize_samples does
+                return false;
+            }
+            sp--;
+            if(sp < kMaxFrames) load_frame<kAhead>(c, pix, sp, F);
+            else F.ahead = 0u;
+            step = resume<kAhead>(c, F, P, out, pix, sp);
+            fresh = false;
         }
-        sp--;
-        if(sp < kMaxFrames) load_frame(c, pix, sp, F);
-        step = resume(c, F, P, out);
-        fresh = false;
     }
 }
 
@@ -954,7 +1089,7 @@ __device__ __forceinline__ HitRec load_hit(const float* hits, size_t n, uint32_t
 // Shades queue entries [base, base + 64) of queue `cur` (one wave, one lane
 // per entry), appending the emitted rays to the other queue with one atomic
 // per wave.
-template<bool kNextSample>
+template<bool kNextSample, bool kAhead>
 __device__ __forceinline__ void shade_wave(const ShadeParams& p, const Ctx& c, int cur, uint32_t count, uint32_t base, int lane,
                                            uint64_t ltMask)
 {
@@ -976,7 +1111,7 @@ __device__ __forceinline__ void shade_wave(const ShadeParams& p, const Ctx& c, i
             Payload P;
             int sp, sample;
             load_state(p, pix, P, sp, sample);
-            emit = advance_pixel<kNextSample>(c, pix, flags, O, D, h, P, sp, sample, out);
+            emit = advance_pixel<kNextSample, kAhead>(c, pix, flags, O, D, h, P, sp, sample, out);
             if(emit) store_state(p, pix, P, sp, sample);
         }
         // append the emitted rays to the next queue, one atomic per wave
@@ -990,17 +1125,19 @@ __device__ __forceinline__ void shade_wave(const ShadeParams& p, const Ctx& c, i
     }
 }
 
-// Wavefront shading pass over the rays traced by the preceding traversal pass.
-template<bool kNextSample>
-__global__ __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_eu(kNextSample ? RGRT_SHADE_WAVES : RGRT_SHADE1_WAVES))) void k_shade(ShadeParams p, int cur)
+// Wavefront shading pass over the rays traced by the preceding traversal
+// pass; `ahead`: a traversal pass follows, so rays may be queued ahead for it.
+template<bool kNextSample, bool kAhead>
+__global__ __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_eu(kNextSample ? RGRT_SHADE_WAVES : kAhead ? RGRT_SHADE_AHEAD_WAVES : RGRT_SHADE1_WAVES))) void k_shade(ShadeParams p, int cur, int ahead)
 {
     const uint32_t count = p.st.counters[cur];
     const int lane = threadIdx.x & 63;
     const uint64_t ltMask = lane == 0 ? 0ull : ((~0ull) >> (64 - lane));
-    const Ctx c{p, f3(p.ubo.lightDir[0], p.ubo.lightDir[1], p.ubo.lightDir[2]), p.ubo.maxRecursions, 0u};
+    const Ctx c{p, f3(p.ubo.lightDir[0], p.ubo.lightDir[1], p.ubo.lightDir[2]), p.ubo.maxRecursions, 0u,
+                ahead ? p.st.counters + kAheadCountWord + (1 - cur) : nullptr};
     const uint32_t stride = gridDim.x * blockDim.x;
     for(uint32_t base = blockIdx.x * blockDim.x + (threadIdx.x & ~63u); base < count; base += stride)
-        shade_wave<kNextSample>(p, c, cur, count, base, lane, ltMask);
+        shade_wave<kNextSample, kAhead>(p, c, cur, count, base, lane, ltMask);
 }
 
 // Scene of a batch that chunk k (64 queue entries) belongs to, from the
@@ -1044,8 +1181,8 @@ __global__ __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_eu(kNe
         const int s = __builtin_amdgcn_readfirstlane(chunk_scene(chunkEnd, numScenes, k, lane));
         const ShadeParams& p = ps[s];
         const uint32_t first = s ? chunkEnd[s - 1] : 0u;
-        const Ctx c{p, f3(p.ubo.lightDir[0], p.ubo.lightDir[1], p.ubo.lightDir[2]), p.ubo.maxRecursions, 0u};
-        shade_wave<kNextSample>(p, c, cur, p.st.counters[cur], (k - first) * 64u, lane, ltMask);
+        const Ctx c{p, f3(p.ubo.lightDir[0], p.ubo.lightDir[1], p.ubo.lightDir[2]), p.ubo.maxRecursions, 0u, nullptr};
+        shade_wave<kNextSample, false>(p, c, cur, p.st.counters[cur], (k - first) * 64u, lane, ltMask);
     }
 }
 
@@ -1059,7 +1196,7 @@ constexpr int kDrainSpill = 368; // see traverse.h: 16 + 368 >= 381
 // the queue (one atomic per wave, a ballot to hand out the entries). The
 // recursion tail thus costs the longest remaining chain of one pixel rather
 // than one launch per recursion step.
-template<bool kNextSample, typename Stack>
+template<bool kNextSample, bool kAhead, typename Stack>
 __device__ __forceinline__ void drain_scene(const ShadeParams& p, const TraceScene& sc, int cur, Stack& stack)
 {
     const uint32_t count = p.st.counters[cur];
@@ -1068,7 +1205,7 @@ __device__ __forceinline__ void drain_scene(const ShadeParams& p, const TraceSce
     uint32_t* fetch = p.st.counters + 2 + cur;
     const int lane = threadIdx.x & 63;
     const uint64_t ltMask = lane == 0 ? 0ull : ((~0ull) >> (64 - lane));
-    const Ctx c{p, f3(p.ubo.lightDir[0], p.ubo.lightDir[1], p.ubo.lightDir[2]), p.ubo.maxRecursions, 0u};
+    const Ctx c{p, f3(p.ubo.lightDir[0], p.ubo.lightDir[1], p.ubo.lightDir[2]), p.ubo.maxRecursions, 0u, nullptr};
     bool active = false;
     bool exhausted = false;
     uint32_t pix = 0, flags = 0;
@@ -1110,7 +1247,7 @@ __device__ __forceinline__ void drain_scene(const ShadeParams& p, const TraceSce
             const HitRec h = traverse<RGRT_INST_EVERY>(sc, r, (flags >> kMaskShift) & 0xffu, stack);
             ++traced;
             OutRay out;
-            if(advance_pixel<kNextSample>(c, pix, flags, f3(r.ox, r.oy, r.oz), f3(r.dx, r.dy, r.dz), h, P, sp, sample, out)) {
+            if(advance_pixel<kNextSample, kAhead>(c, pix, flags, f3(r.ox, r.oy, r.oz), f3(r.dx, r.dy, r.dz), h, P, sp, sample, out)) {
                 r.ox = out.o.x;
                 r.oy = out.o.y;
                 r.oz = out.o.z;
@@ -1131,15 +1268,15 @@ __device__ __forceinline__ void drain_scene(const ShadeParams& p, const TraceSce
     if(lane == 0 && traced) atomicAdd(reinterpret_cast<unsigned long long*>(p.st.counters + 4), (unsigned long long)traced);
 }
 
-template<bool kNextSample>
-__global__ __launch_bounds__(kDrainBlock) __attribute__((amdgpu_waves_per_eu(kNextSample ? RGRT_DRAIN_WAVES : RGRT_DRAIN1_WAVES))) void k_drain(ShadeParams p, TraceScene sc, int cur, int32_t* __restrict__ spillBase)
+template<bool kNextSample, bool kAhead>
+__global__ __launch_bounds__(kDrainBlock) __attribute__((amdgpu_waves_per_eu(kNextSample ? RGRT_DRAIN_WAVES : kAhead ? RGRT_DRAIN_AHEAD_WAVES : RGRT_DRAIN1_WAVES))) void k_drain(ShadeParams p, TraceScene sc, int cur, int32_t* __restrict__ spillBase)
 {
     __shared__ int32_t ldsStack[kDrainLdsStack * kDrainBlock];
     const uint32_t gtid = blockIdx.x * kDrainBlock + threadIdx.x;
     __shared__ float boxRay[kBoxRayWords * kDrainBlock];
     TraversalStack<kDrainLdsStack, kDrainBlock, kDrainSpill> stack{ldsStack, spillBase + (size_t)gtid * kDrainSpill,
                                                                    (int)threadIdx.x, boxRay};
-    drain_scene<kNextSample>(p, sc, cur, stack);
+    drain_scene<kNextSample, kAhead>(p, sc, cur, stack);
 }
 
 // Drain of a whole batch: every wave drains the scenes in order, moving to
@@ -1158,7 +1295,7 @@ __global__ __launch_bounds__(kDrainBlock) __attribute__((amdgpu_waves_per_eu(kNe
                                                                    (int)threadIdx.x, boxRay};
     for(int s = 0; s < numScenes; ++s) {
         const TraceScene sc = scs[s];
-        drain_scene<kNextSample>(ps[s], sc, cur, stack);
+        drain_scene<kNextSample, false>(ps[s], sc, cur, stack);
     }
 }
 
@@ -1188,12 +1325,12 @@ bool run_one_sample(const ShadeParams& p)
     return p.st.groups >= (uint32_t)std::max(1, p.ubo.numSamples);
 }
 
-void launch_shade(hipStream_t s, const ShadeParams& p, int cur, uint32_t gridBlocks)
+void launch_shade(hipStream_t s, const ShadeParams& p, int cur, uint32_t gridBlocks, bool ahead)
 {
-    if(run_one_sample(p))
-        k_shade<false><<<gridBlocks, kShadeBlock, 0, s>>>(p, cur);
-    else
-        k_shade<true><<<gridBlocks, kShadeBlock, 0, s>>>(p, cur);
+    const bool one = run_one_sample(p);
+    if(one && p.aheadOn) k_shade<false, true><<<gridBlocks, kShadeBlock, 0, s>>>(p, cur, ahead ? 1 : 0);
+    else if(one) k_shade<false, false><<<gridBlocks, kShadeBlock, 0, s>>>(p, cur, 0);
+    else k_shade<true, false><<<gridBlocks, kShadeBlock, 0, s>>>(p, cur, 0);
 }
 
 uint32_t drain_spill_words_per_thread() { return kDrainSpill; }
@@ -1201,10 +1338,10 @@ uint32_t drain_block_size() { return kDrainBlock; }
 
 void launch_drain(hipStream_t s, const ShadeParams& p, const TraceScene& sc, int cur, uint32_t gridBlocks, int32_t* spill)
 {
-    if(run_one_sample(p))
-        k_drain<false><<<gridBlocks, kDrainBlock, 0, s>>>(p, sc, cur, spill);
-    else
-        k_drain<true><<<gridBlocks, kDrainBlock, 0, s>>>(p, sc, cur, spill);
+    const bool one = run_one_sample(p);
+    if(one && p.aheadOn) k_drain<false, true><<<gridBlocks, kDrainBlock, 0, s>>>(p, sc, cur, spill);
+    else if(one) k_drain<false, false><<<gridBlocks, kDrainBlock, 0, s>>>(p, sc, cur, spill);
+    else k_drain<true, false><<<gridBlocks, kDrainBlock, 0, s>>>(p, sc, cur, spill);
 }
 
 void launch_shade_multi(hipStream_t s, const ShadeParams* ps, int numScenes, int cur, uint32_t gridBlocks, bool oneSample)

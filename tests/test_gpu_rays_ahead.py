@@ -1,0 +1,51 @@
+"""Rays queued ahead (a hit's reflection and refraction rays traced beside its
+shadow ray): frames with one sample per slot take that path, frames whose
+slots run their samples one after another do not, and both give the same
+images and ray counts bit for bit, wherever the wavefront passes end and the
+drain takes over. The scene's materials reflect and refract at once, so a
+reflection's subtree changes the index of refraction a ray queued ahead had
+assumed, and closed meshes give total internal reflection."""
+import numpy as np
+import pytest
+
+from helpers import gpu_context
+from raygun_amd import procgen, rgrt
+
+pytestmark = pytest.mark.gpu
+
+
+def glass_scene(w, h, depth):
+    setup = procgen.config5(w, h, tris_per_mesh=2_000, num_instances=40, num_samples=2)
+    setup.max_recursions = depth
+    rng = np.random.default_rng(4)
+    for model in setup.scene.models():
+        m = model.materials
+        m["reflectivity"] = rng.uniform(0.2, 0.9)
+        m["transparency"] = rng.uniform(0.3, 0.9)
+        m["ior"] = rng.uniform(1.1, 1.8)
+        m["rayConsumption"] = rng.integers(1, 3)
+    return setup
+
+
+@pytest.mark.parametrize("passes", [0, 1, 2, 3, 64])
+@pytest.mark.parametrize("stochastic", [False, True])
+def test_rays_ahead_change_no_image(passes, stochastic):
+    print(f"[case] rays ahead passes={passes} stochastic={stochastic}", flush=True)
+    setup = glass_scene(121, 67, 4)
+    ctx, _ = gpu_context(setup, flags=rgrt.CFG_FP32_RADIANCE)
+    try:
+        if stochastic:
+            ctx.set_sampling(rgrt.SAMPLING_STOCHASTIC, 9)
+        ctx.set_tuning(wavefrontPasses=passes)
+        seen = []
+        for groups in (1, 2):  # samples one after another (plain), side by side (rays ahead)
+            ctx.set_sample_groups(groups)
+            ctx.render(True)
+            images = [ctx.read_image(k) for k in (rgrt.IMAGE_BASE_F32, rgrt.IMAGE_ROUGH_F32, rgrt.IMAGE_FINAL)]
+            s = ctx.stats()
+            seen.append((images, (s["rays"], s["skyLookups"], s["zeroDirRays"])))
+        assert seen[0][1] == seen[1][1]
+        for a, b in zip(seen[0][0], seen[1][0]):
+            assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
+    finally:
+        ctx.close()
