@@ -11,17 +11,17 @@ namespace {
 
 constexpr int kTraceBlock = 256;
 constexpr int kLdsStack = 16;
-constexpr int kSpill = 368; // with the 16 LDS entries: the 381-entry worst case of two wide LBVH levels
+constexpr int kSpill = 368; // with the 16 LDS entries: the 382-entry worst case of two wide LBVH levels
 
 // Wavefront trace pass: rays [0, count) of queue `cur` -> hit records, and
 // the rays queued ahead -> the frames that will need their hits. Waves fetch
 // 64 rays at a time from a global counter (persistent grid).
 // Waves per SIMD the traversal pass is compiled for: the register budget is
-// 512 / waves VGPRs. At 7 waves (73) nine registers spill in the loop: a
-// 1080p frame over 2M triangles takes 8.92 ms against 8.75 at 6 waves, 3,000
-// small instances 3.74 against 3.62 ms.
+// 512 / waves VGPRs, its loop needs 94. At 6 waves (80, seven spilled in the
+// loop) 3,000 small instances take 3.62 ms against 3.43 at 5, a 640x360 frame
+// 0.465 against 0.447, larger frames the same.
 #ifndef RGRT_TRACE_WAVES
-#define RGRT_TRACE_WAVES 6
+#define RGRT_TRACE_WAVES 5
 #endif
 
 template<bool kAhead>

@@ -17,7 +17,8 @@
 // a wave's pushes hit distinct banks) and spills to a per-thread global
 // region beyond that depth. A wide node pushes at most 3 entries and an
 // LBVH is at most 63 levels deep, so two levels need at most
-// 2 x (3 x 63 + 1) + 1 = 381 entries: kLdsStack + spill = 384.
+// 2 x (3 x 63 + 1) + 1 = 381 entries and the bottom marker: kLdsStack + spill
+// = 384.
 #pragma once
 
 #include "rgrt_device.h"
@@ -53,6 +54,34 @@ struct BoxRay {
 
 __device__ __forceinline__ float pow2i(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
 
+// The hardware's three-operand maximum and minimum (fmaxf and fminf would
+// first quiet operands the compiler cannot prove quiet; the box test never
+// meets a NaN from finite rays, and one only culls or not).
+__device__ __forceinline__ float max3f(float a, float b, float c)
+{
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float min3f(float a, float b, float c)
+{
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float max2f(float a, float b)
+{
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float min2f(float a, float b)
+{
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
 __device__ __forceinline__ void cswap(float& ta, int32_t& ra, float& tb, int32_t& rb)
 {
     const bool sw = tb < ta;
@@ -86,8 +115,8 @@ __device__ __forceinline__ float qbox_enter(uint32_t nx, uint32_t fx, uint32_t n
     const float xn = __builtin_fmaf((float)((nx >> sh) & 0xffu), ax, bxn), xf = __builtin_fmaf((float)((fx >> sh) & 0xffu), ax, bxf);
     const float yn = __builtin_fmaf((float)((ny >> sh) & 0xffu), ay, byn), yf = __builtin_fmaf((float)((fy >> sh) & 0xffu), ay, byf);
     const float zn = __builtin_fmaf((float)((nz >> sh) & 0xffu), az, bzn), zf = __builtin_fmaf((float)((fz >> sh) & 0xffu), az, bzf);
-    const float n = fmaxf(fmaxf(xn, yn), fmaxf(zn, tmin));
-    const float f = fminf(fminf(xf, yf), fminf(zf, tmax));
+    const float n = max3f(xn, yn, max2f(zn, tmin));
+    const float f = min3f(xf, yf, min2f(zf, tmax));
     return n <= f * 1.0000008f ? n : INFINITY;
 }
 
@@ -103,7 +132,7 @@ __device__ __forceinline__ int32_t visit_wide(const u32x4 v0, const u32x4 v1, co
 {
     const int4 ch = make_int4((int)v3.x, (int)v3.y, (int)v3.z, (int)v3.w);
     const int ex = (int)(int8_t)(v0.w & 0xffu), ey = (int)(int8_t)((v0.w >> 8) & 0xffu), ez = (int)(int8_t)((v0.w >> 16) & 0xffu);
-    const float ax = pow2i(ex) * br.ix, ay = pow2i(ey) * br.iy, az = pow2i(ez) * br.iz;
+    const float ax = __builtin_ldexpf(br.ix, ex), ay = __builtin_ldexpf(br.iy, ey), az = __builtin_ldexpf(br.iz, ez);
     const float bx = (__uint_as_float(v0.x) - br.ox) * br.ix;
     const float by = (__uint_as_float(v0.y) - br.oy) * br.iy;
     const float bz = (__uint_as_float(v0.z) - br.oz) * br.iz;
@@ -120,7 +149,7 @@ __device__ __forceinline__ int32_t visit_wide(const u32x4 v0, const u32x4 v1, co
     const float e1 = qbox_enter(nx, fx, ny, fy, nz, fz, 1, ax, bxn, bxf, ay, byn, byf, az, bzn, bzf, tmin, tbest);
     const float e2 = qbox_enter(nx, fx, ny, fy, nz, fz, 2, ax, bxn, bxf, ay, byn, byf, az, bzn, bzf, tmin, tbest);
     const float e3 = qbox_enter(nx, fx, ny, fy, nz, fz, 3, ax, bxn, bxf, ay, byn, byf, az, bzn, bzf, tmin, tbest);
-    float t0 = ch.x != kEmptyChild ? e0 : INFINITY;
+    float t0 = e0; // a node has a first child
     float t1 = ch.y != kEmptyChild ? e1 : INFINITY;
     float t2 = ch.z != kEmptyChild ? e2 : INFINITY;
     float t3 = ch.w != kEmptyChild ? e3 : INFINITY;
@@ -130,9 +159,18 @@ __device__ __forceinline__ int32_t visit_wide(const u32x4 v0, const u32x4 v1, co
     cswap(t0, r0, t2, r2);
     cswap(t1, r1, t3, r3);
     cswap(t1, r1, t2, r2);
-    if(t3 != INFINITY) stack.push(r3);
-    if(t2 != INFINITY) stack.push(r2);
-    if(t1 != INFINITY) stack.push(r1);
+    // (with room for three in LDS, all three are written where the next entry
+    // goes and the top moves past the hit ones: no branches)
+    if(stack.lds_has_room(3)) {
+        stack.push_lds_if(r3, t3 != INFINITY);
+        stack.push_lds_if(r2, t2 != INFINITY);
+        stack.push_lds_if(r1, t1 != INFINITY);
+    }
+    else {
+        if(t3 != INFINITY) stack.push(r3);
+        if(t2 != INFINITY) stack.push(r2);
+        if(t1 != INFINITY) stack.push(r1);
+    }
     return t0 != INFINITY ? r0 : kEmptyChild;
 }
 
@@ -257,9 +295,23 @@ struct TraversalStack {
         else if(sp < kLdsStack + kSpillWords) spill[sp - kLdsStack] = v;
         ++sp;
     }
+    // Entries are rarely past the LDS part, so the wave asks once for all its
+    // lanes here instead of branching in each push and pop.
+    __device__ __forceinline__ bool lds_has_room(int n) const { return __ballot(sp > kLdsStack - n) == 0ull; }
+    __device__ __forceinline__ void push_lds_if(int32_t v, bool c)
+    {
+        lds[sp * kBlock + tid] = v;
+        sp += c ? 1 : 0;
+    }
+    __device__ __forceinline__ void push_lds(int32_t v)
+    {
+        lds[sp * kBlock + tid] = v;
+        ++sp;
+    }
     __device__ __forceinline__ int32_t pop()
     {
         --sp;
+        if(__ballot(sp >= kLdsStack) == 0ull) return lds[sp * kBlock + tid];
         if(sp < kLdsStack) return lds[sp * kBlock + tid];
         if(sp < kLdsStack + kSpillWords) return spill[sp - kLdsStack];
         return kSentinel;
@@ -291,26 +343,26 @@ struct Traversal {
     int32_t ref;
     uint32_t cullMask;
     uint32_t curInst;
-    uint32_t nodeCap;    // nodes of the tree being walked
-    uint32_t leafCap;    // its leaves
-    uint32_t leafStride; // bytes of a leaf record
-    bool inBlas;
+    uint32_t nodeLast;   // last node of the tree being walked
+    uint32_t leafLast;   // its last leaf
+    uint32_t leafStride; // bytes of a leaf record: an instance's in the TLAS, a triangle's in a BLAS
     HitRec h;
 };
 
 // Every index a traversal step uses is checked against the table it
 // indexes; a bad one (a corrupt tree or table) ends the ray as a miss and
-// raises a sticky flag that the host turns into an error.
-__device__ __noinline__ void trav_error(const TraceScene& sc, uint32_t flag) { atomicOr(sc.errors, flag); }
+// raises a sticky flag that the host turns into an error. The flag waits
+// above the cull mask's 8 bits until the loop has ended.
+constexpr uint32_t kTravErrShift = 16u;
+constexpr int32_t kDone = (int32_t)0x80000001; // below every leaf: a leaf index is below 2^31 - 2
 
 __device__ __forceinline__ void enter_tlas(Traversal& T, const TraceScene& sc)
 {
     T.nodes = reinterpret_cast<const char*>(sc.tlasNodes);
     T.leaves = reinterpret_cast<const char*>(sc.instances);
-    T.nodeCap = sc.tlasNodeCap;
-    T.leafCap = sc.numInstances;
+    T.nodeLast = sc.tlasNodeCap - 1u;
+    T.leafLast = sc.numInstances - 1u;
     T.leafStride = sizeof(DevInstance);
-    T.inBlas = false;
 }
 
 // Starts a ray at the TLAS root; false if there is nothing to traverse.
@@ -328,6 +380,7 @@ __device__ __forceinline__ bool trav_begin(Traversal& T, const TraceScene& sc, c
     T.ref = 0;
     T.cullMask = cullMask;
     stack.sp = 0;
+    stack.push_lds(kDone);
     T.wix = safe_rcp(ray.dx);
     T.wiy = safe_rcp(ray.dy);
     T.wiz = safe_rcp(ray.dz);
@@ -337,7 +390,7 @@ __device__ __forceinline__ bool trav_begin(Traversal& T, const TraceScene& sc, c
 
 // One iteration of a wave's loop: a wide node, a triangle or an instance
 // leaf, and the pop after it, which takes the return to the TLAS with it.
-// Returns false once the ray is finished (T.h holds the closest hit).
+// T.ref is kDone once the ray is finished (T.h holds the closest hit).
 //
 // A wave runs every kind of step its lanes need in each iteration and, if
 // each kind loads its own record, waits for one memory latency after the
@@ -350,34 +403,40 @@ __device__ __forceinline__ bool trav_begin(Traversal& T, const TraceScene& sc, c
 // one iteration, each with its own loads, needs a fifth fewer iterations
 // and was slower on those (0.687, 9.41 ms).
 //
+// Scalar instructions cost a wave as much as vector ones here (keeping three
+// direction-sign masks across the loop added 108 of them and cost 15%), so
+// nothing that merges in the loop is a lane mask: what the lane is at follows
+// from T.ref and T.leafStride, the stack's bottom entry ends the ray, a bad
+// index is clamped and flagged without a branch, and the LDS part of the
+// stack is checked once per node for the wave. The same rays 0.638 -> 0.575
+// ms, 3,000 small instances 3.62 -> 3.43 ms.
+//
 // An instance entry is rare (some 8% of a ray's steps) and costs as much as
 // a node visit, so it is taken only in iterations `iter` that are multiples
 // of kInstEvery; a lane that reaches one in another iteration waits with its
 // state unchanged. `iter` must count the wave's iterations (all lanes start
 // the ray together). Every ray takes the same steps in the same order
-// whatever kInstEvery is. Measured on the frame and the rays above: every
-// iteration 9.62 and 0.672 ms, every second 8.92 and 0.640, every fourth
-// 8.78 and 0.638; 3,000 small instances 4.08, 3.74 and 3.76 ms.
+// whatever kInstEvery is. Measured on that frame and 3,000 small instances:
+// every second iteration 8.69 and 3.43 ms, every fourth 8.51 and 3.49; every
+// iteration was slower than both on each (9.62 against 8.92 and 8.78, 4.08
+// against 3.74 and 3.76 before the loop's scalar work was cut).
 template<int kInstEvery = 1, typename Stack>
-__device__ __forceinline__ bool trav_step(Traversal& T, const TraceScene& sc, Stack& stack, uint32_t iter = 0)
+__device__ __forceinline__ void trav_step(Traversal& T, const TraceScene& sc, Stack& stack, uint32_t iter = 0)
 {
     const bool isNode = T.ref >= 0;
-    if(kInstEvery > 1 && iter % kInstEvery != 0u && !isNode && !T.inBlas) return true; // an entry of a later iteration
+    const bool inTlas = T.leafStride == sizeof(DevInstance);
+    if(kInstEvery > 1 && iter % kInstEvery != 0u && !isNode && inTlas) return; // an entry of a later iteration
     const uint32_t idx = (uint32_t)(isNode ? T.ref : ~T.ref);
-    if(idx >= (isNode ? T.nodeCap : T.leafCap)) {
-        trav_error(sc, isNode ? kTravErrNode : T.inBlas ? kTravErrTriangle : kTravErrInstance);
-        T.h.inst = kNoHit;
-        return false;
-    }
+    const uint32_t last = isNode ? T.nodeLast : T.leafLast;
+    if(idx > last) T.cullMask |= (isNode ? kTravErrNode : inTlas ? kTravErrInstance : kTravErrTriangle) << kTravErrShift;
     // one fetch for whatever the lane is at
-    const u32x4* ip = reinterpret_cast<const u32x4*>((isNode ? T.nodes : T.leaves) + (uint64_t)idx * (isNode ? 64u : T.leafStride));
+    const u32x4* ip = reinterpret_cast<const u32x4*>((isNode ? T.nodes : T.leaves) + (uint64_t)min(idx, last) * (isNode ? 64u : T.leafStride));
     const u32x4 v0 = ld_global16(ip), v1 = ld_global16(ip + 1), v2 = ld_global16(ip + 2), v3 = ld_global16(ip + 3);
-    bool pop = true;
     if(isNode) {
         T.ref = visit_wide(v0, v1, v2, v3, stack.box_ray(), T.ray.tmin, T.tbest, stack);
-        pop = T.ref == kEmptyChild;
     }
-    else if(T.inBlas) { // a triangle
+    else if(!inTlas) { // a triangle
+        T.ref = kEmptyChild;
         Tri tri;
         tri.v0x = __uint_as_float(v0.x);
         tri.v0y = __uint_as_float(v0.y);
@@ -399,15 +458,12 @@ __device__ __forceinline__ bool trav_step(Traversal& T, const TraceScene& sc, St
         }
     }
     else { // an instance: v3 = blas, mask, position, customIndex
-        if(v3.x >= sc.numBlas) {
-            trav_error(sc, kTravErrBlas);
-            T.h.inst = kNoHit;
-            return false;
-        }
-        const u32x4* bp = reinterpret_cast<const u32x4*>(sc.blas + v3.x);
+        T.ref = kEmptyChild;
+        if(v3.x >= sc.numBlas) T.cullMask |= kTravErrBlas << kTravErrShift;
+        const u32x4* bp = reinterpret_cast<const u32x4*>(sc.blas + min(v3.x, sc.numBlas - 1u));
         const u32x4 b0 = ld_global16(bp);     // nodes, tris
         const uint32_t numFaces = ld_global8(bp + 1).x;
-        if((v3.y & T.cullMask) != 0u && numFaces > 0u) {
+        if((v3.y & T.cullMask & 0xffu) != 0u && numFaces > 0u) {
             const float w[12] = {__uint_as_float(v0.x), __uint_as_float(v0.y), __uint_as_float(v0.z), __uint_as_float(v0.w),
                                  __uint_as_float(v1.x), __uint_as_float(v1.y), __uint_as_float(v1.z), __uint_as_float(v1.w),
                                  __uint_as_float(v2.x), __uint_as_float(v2.y), __uint_as_float(v2.z), __uint_as_float(v2.w)};
@@ -420,25 +476,21 @@ __device__ __forceinline__ bool trav_step(Traversal& T, const TraceScene& sc, St
             // the copy of the triangles in this ray's axis order
             T.leaves = reinterpret_cast<const char*>((uint64_t)b0.z | ((uint64_t)b0.w << 32)) + (uint64_t)rot * numFaces * sizeof(Tri);
             T.leafStride = sizeof(Tri);
-            T.inBlas = true;
             T.curInst = v3.z;
-            T.leafCap = numFaces;
-            T.nodeCap = numFaces > 2u ? numFaces - 1u : 1u;
+            T.leafLast = numFaces - 1u;
+            T.nodeLast = numFaces > 2u ? numFaces - 2u : 0u;
             T.ref = 0;
-            pop = false;
         }
     }
-    if(pop) {
-        if(stack.sp == 0) return false;
-        T.ref = stack.pop();
+    if(T.ref == kEmptyChild) {
+        T.ref = stack.pop(); // the bottom entry is kDone
         if(T.ref == kSentinel) { // back to the TLAS and its next entry (never a sentinel)
-            if(stack.sp == 0) return false;
             T.ref = stack.pop();
             enter_tlas(T, sc);
             stack.set_box_ray(T.ray.ox, T.ray.oy, T.ray.oz, T.wix, T.wiy, T.wiz);
         }
     }
-    return true;
+    if(T.cullMask >> kTravErrShift) T.ref = kDone;
 }
 
 // Iterations between a wave's instance entries (trav_step): the schedule of
@@ -457,7 +509,14 @@ __device__ HitRec traverse(const TraceScene& sc, const RayIn& ray, uint32_t cull
     Traversal T;
     if(trav_begin(T, sc, ray, cullMask, stack)) {
         for(uint32_t guard = 0; guard < (1u << 26); ++guard)
-            if(!trav_step<kInstEvery>(T, sc, stack, guard)) break;
+        {
+            trav_step<kInstEvery>(T, sc, stack, guard);
+            if(T.ref == kDone) break;
+        }
+    }
+    if(T.cullMask >> kTravErrShift) {
+        atomicOr(sc.errors, T.cullMask >> kTravErrShift);
+        T.h.inst = kNoHit;
     }
     T.h.t = T.h.inst != kNoHit ? T.tbest : 0.0f;
     return T.h;

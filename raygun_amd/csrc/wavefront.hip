@@ -1188,7 +1188,7 @@ __global__ __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_eu(kNe
 
 constexpr int kDrainBlock = 256;
 constexpr int kDrainLdsStack = 16;
-constexpr int kDrainSpill = 368; // see traverse.h: 16 + 368 >= 381
+constexpr int kDrainSpill = 368; // see traverse.h: 16 + 368 >= 382
 
 // Drain: finishes every pixel still in flight after the wavefront passes.
 // Each lane takes a queued ray, traces and shades it, and keeps tracing that
