@@ -728,9 +728,9 @@ rgrt_status do_trace(rgrt_ctx* c)
     if(!drained && it == maxIters) {
         // all pixels must be done after the bound; check the last count
         check(hipStreamSynchronize(s));
-        uint32_t remaining = 0;
-        check(hipMemcpy(&remaining, c->st.counters + cur, 4, hipMemcpyDeviceToHost));
-        if(remaining) return fail(c, RGRT_ERR_HIP, "rgrt_trace: ray queue did not drain within the recursion bound");
+        uint32_t counts[kCounterBlock];
+        check(hipMemcpy(counts, c->st.counters, sizeof(counts), hipMemcpyDeviceToHost));
+        if(counts[cur] + counts[kQueueBackWord + cur]) return fail(c, RGRT_ERR_HIP, "rgrt_trace: ray queue did not drain within the recursion bound");
     }
     launch_finalize_samples(s, p);
     if(timing) check(hipEventRecord(c->evRtOnlyEnd, s));

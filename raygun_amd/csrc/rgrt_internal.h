@@ -150,8 +150,42 @@ struct WavefrontState {
     float* rays[2] = {nullptr, nullptr}; // [kRayWords][npix]
     float* hits = nullptr;    // [kHitWords][npix]
     float* ahead = nullptr;   // [kAheadWords][kAheadPerSlot * npix]: rays traced ahead by the next pass
-    uint32_t* counters = nullptr; // [0..1] queue counts, [2..3] fetch, [4..9] stats (u64 pairs), [10..11] rays ahead, [12] traversal errors
+    // [0..1] rays at the front of queue 0, 1, [2..3] fetch, [4..9] stats (u64 pairs), [10..11] rays ahead, [12]
+    // traversal errors, [13..14] rays at the back of queue 0, 1
+    uint32_t* counters = nullptr;
     float* lum2 = nullptr;        // [npix]: sum of squared sample luminances (stochastic sampling)
+};
+
+constexpr int kQueueBackWord = 13;
+
+// Queue `cur` of a frame (or band): in frames of more than kSortedSlots slots
+// shadow rays fill it from the front and all others from the back, so a wave's
+// 64 entries are of one sort (shadow rays of neighbouring pixels run in
+// parallel, and their shading takes one path): 4K at 4 samples 94.2 -> 91.4
+// ms, 1080p over 2M triangles 8.62 -> 8.49. Smaller frames, whose passes wait
+// on their slowest rays, keep one end (split, 960x540 over 3,000 instances
+// measured 3.44 -> 3.47 ms, 640x360 0.456 -> 0.459). Work on it is cut into
+// 64-entry chunks, the front's then the back's.
+constexpr uint32_t kSortedSlots = 1u << 20;
+struct QueueSpan {
+    uint32_t front, back, frontChunks, chunks, size;
+    __device__ __forceinline__ QueueSpan(const WavefrontState& st, int cur)
+    {
+        front = st.counters[cur];
+        back = st.counters[kQueueBackWord + cur];
+        frontChunks = (front + 63u) / 64u;
+        chunks = frontChunks + (back + 63u) / 64u;
+        size = st.npix;
+    }
+    __device__ __forceinline__ uint32_t count() const { return front + back; }
+    // Queue position of a lane of chunk k; false past its end.
+    __device__ __forceinline__ bool entry(uint32_t k, uint32_t lane, uint32_t& i) const
+    {
+        const bool isBack = k >= frontChunks;
+        const uint32_t j = (isBack ? k - frontChunks : k) * 64u + lane;
+        i = isBack ? size - 1u - j : j;
+        return j < (isBack ? back : front);
+    }
 };
 
 struct Images {

@@ -34,15 +34,16 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(RGR
     float* __restrict__ hits = st.hits;
     const size_t npix = st.npix;
     const size_t aheadCap = npix * kAheadPerSlot;
-    const uint32_t count = counters[cur];
+    const QueueSpan queue(st, cur);
     const uint32_t ahead = kAhead ? (uint32_t)min((size_t)counters[kAheadCountWord + cur], aheadCap) : 0u;
     if(blockIdx.x == 0 && threadIdx.x == 0) {
-        *hostSlot = count + ahead; // host-visible: lets the host stop once the queues drain
-        counters[1 - cur] = 0;     // the output queues of the shading pass that follows
+        *hostSlot = queue.count() + ahead; // host-visible: lets the host stop once the queues drain
+        counters[1 - cur] = 0;             // the output queues of the shading pass that follows
+        counters[kQueueBackWord + (1 - cur)] = 0;
         counters[kAheadCountWord + (1 - cur)] = 0;
         counters[2 + (1 - cur)] = 0; // the fetch counter of the next traversal pass
         // ray statistics (64-bit) at counters[4..5]
-        atomicAdd(reinterpret_cast<unsigned long long*>(counters + 4), (unsigned long long)count + ahead);
+        atomicAdd(reinterpret_cast<unsigned long long*>(counters + 4), (unsigned long long)queue.count() + ahead);
     }
     const int lane = threadIdx.x & 63;
     const uint32_t gtid = blockIdx.x * kTraceBlock + threadIdx.x;
@@ -54,13 +55,12 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(RGR
     // static share are fetched from a counter, so a pass with fewer rays than
     // the grid has lanes does no atomics at all.
     const uint32_t wavesInGrid = gridDim.x * (kTraceBlock / 64);
-    const uint32_t mainChunks = (count + 63u) / 64u;
-    const uint32_t chunks = mainChunks + (ahead + 63u) / 64u;
+    const uint32_t chunks = queue.chunks + (ahead + 63u) / 64u;
     uint32_t k = blockIdx.x * (kTraceBlock / 64) + (threadIdx.x >> 6);
     while(k < chunks) {
-        const bool isAhead = kAhead && k >= mainChunks;
-        const uint32_t i = (isAhead ? k - mainChunks : k) * 64u + lane;
-        if(i < (isAhead ? ahead : count)) {
+        const bool isAhead = kAhead && k >= queue.chunks;
+        uint32_t i = isAhead ? (k - queue.chunks) * 64u + lane : 0u;
+        if(isAhead ? i < ahead : queue.entry(k, lane, i)) {
             RayIn r;
             uint32_t mask, slot = 0;
             if(isAhead) {
@@ -126,8 +126,9 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(RGR
     if(threadIdx.x < 64) {
         uint32_t count = 0, v = 0;
         if(lane < numScenes) {
-            count = ps[lane].st.counters[cur];
-            v = (count + 63u) / 64u;
+            const QueueSpan queue(ps[lane].st, cur);
+            count = queue.count();
+            v = queue.chunks;
         }
         for(int off = 1; off < 64; off <<= 1) {
             const uint32_t u = __shfl_up(v, off);
@@ -138,6 +139,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(RGR
             if(lane < numScenes) {
                 uint32_t* counters = ps[lane].st.counters;
                 counters[1 - cur] = 0;       // the output queue of the shading pass that follows
+                counters[kQueueBackWord + (1 - cur)] = 0;
                 counters[2 + (1 - cur)] = 0; // the fetch counter of the drain
                 atomicAdd(reinterpret_cast<unsigned long long*>(counters + 4), (unsigned long long)count);
             }
@@ -156,9 +158,8 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(RGR
         const int s = __builtin_amdgcn_readfirstlane(__popcll(__ballot(lane < numScenes && chunkEnd[lane < numScenes ? lane : 0] <= k)));
         const uint32_t first = s ? chunkEnd[s - 1] : 0u;
         const WavefrontState& st = ps[s].st;
-        const uint32_t count = st.counters[cur];
-        const uint32_t i = (k - first) * 64u + (uint32_t)lane;
-        if(i < count) {
+        uint32_t i;
+        if(QueueSpan(st, cur).entry(k - first, (uint32_t)lane, i)) {
             const size_t npix = st.npix;
             const float* __restrict__ rays = st.rays[cur];
             float* __restrict__ hits = st.hits;

@@ -874,6 +874,8 @@ __device__ __forceinline__ void raygen_slot(const ShadeParams& p, uint32_t q)
         uint32_t* c = p.st.counters;
         c[0] = p.st.npix; // queue 0 holds every slot's primary ray
         c[1] = 0;
+        c[kQueueBackWord] = 0;
+        c[kQueueBackWord + 1] = 0;
         c[2] = 0;
         c[3] = 0;
         for(int k = 4; k < 12; ++k) c[k] = 0; // ray / sky / zero-dir counters (u64), rays ahead
@@ -1086,42 +1088,40 @@ __device__ __forceinline__ HitRec load_hit(const float* hits, size_t n, uint32_t
     return h;
 }
 
-// Shades queue entries [base, base + 64) of queue `cur` (one wave, one lane
-// per entry), appending the emitted rays to the other queue with one atomic
+// Shades chunk k of queue `cur` (one wave, one lane per entry), appending the
+// emitted rays to an end of the other queue (QueueSpan), one atomic instruction
 // per wave.
 template<bool kNextSample, bool kAhead>
-__device__ __forceinline__ void shade_wave(const ShadeParams& p, const Ctx& c, int cur, uint32_t count, uint32_t base, int lane,
+__device__ __forceinline__ void shade_wave(const ShadeParams& p, const Ctx& c, int cur, const QueueSpan& queue, uint32_t k, int lane,
                                            uint64_t ltMask)
 {
     const size_t n = p.st.npix;
     const float* __restrict__ rays = p.st.rays[cur];
     float* __restrict__ outRays = p.st.rays[1 - cur];
-    uint32_t* outCount = p.st.counters + (1 - cur);
-    {
-        const uint32_t i = base + lane;
-        bool emit = false;
-        OutRay out;
-        uint32_t pix = 0;
-        if(i < count) {
-            pix = __float_as_uint(rays[8 * n + i]);
-            const uint32_t flags = __float_as_uint(rays[9 * n + i]);
-            const F3 O = f3(rays[0 * n + i], rays[1 * n + i], rays[2 * n + i]);
-            const F3 D = f3(rays[4 * n + i], rays[5 * n + i], rays[6 * n + i]);
-            const HitRec h = load_hit(p.st.hits, n, i);
-            Payload P;
-            int sp, sample;
-            load_state(p, pix, P, sp, sample);
-            emit = advance_pixel<kNextSample, kAhead>(c, pix, flags, O, D, h, P, sp, sample, out);
-            if(emit) store_state(p, pix, P, sp, sample);
-        }
-        // append the emitted rays to the next queue, one atomic per wave
-        const uint64_t m = __ballot(emit);
-        if(m) {
-            uint32_t wbase = 0;
-            if(lane == 0) wbase = atomicAdd(outCount, (uint32_t)__popcll(m));
-            wbase = __shfl(wbase, 0);
-            if(emit) write_ray(outRays, n, wbase + (uint32_t)__popcll(m & ltMask), out, pix, (out.mask << kMaskShift) | out.miss1);
-        }
+    bool emit = false, front = false;
+    OutRay out;
+    uint32_t pix = 0, i;
+    if(queue.entry(k, (uint32_t)lane, i)) {
+        pix = __float_as_uint(rays[8 * n + i]);
+        const uint32_t flags = __float_as_uint(rays[9 * n + i]);
+        const F3 O = f3(rays[0 * n + i], rays[1 * n + i], rays[2 * n + i]);
+        const F3 D = f3(rays[4 * n + i], rays[5 * n + i], rays[6 * n + i]);
+        const HitRec h = load_hit(p.st.hits, n, i);
+        Payload P;
+        int sp, sample;
+        load_state(p, pix, P, sp, sample);
+        emit = advance_pixel<kNextSample, kAhead>(c, pix, flags, O, D, h, P, sp, sample, out);
+        if(emit) store_state(p, pix, P, sp, sample);
+        front = p.st.frameSlots <= kSortedSlots || P.rayType != RT_GENERIC;
+    }
+    const uint64_t toFront = __ballot(emit && front), toBack = __ballot(emit && !front);
+    if(toFront | toBack) {
+        uint32_t base = 0;
+        if(lane < 2)
+            base = atomicAdd(p.st.counters + (lane ? kQueueBackWord : 0) + (1 - cur), (uint32_t)__popcll(lane ? toBack : toFront));
+        const uint32_t f0 = (uint32_t)__builtin_amdgcn_readlane((int)base, 0), b0 = (uint32_t)__builtin_amdgcn_readlane((int)base, 1);
+        const uint32_t at = front ? f0 + (uint32_t)__popcll(toFront & ltMask) : (uint32_t)n - 1u - (b0 + (uint32_t)__popcll(toBack & ltMask));
+        if(emit) write_ray(outRays, n, at, out, pix, (out.mask << kMaskShift) | out.miss1);
     }
 }
 
@@ -1130,14 +1130,14 @@ __device__ __forceinline__ void shade_wave(const ShadeParams& p, const Ctx& c, i
 template<bool kNextSample, bool kAhead>
 __global__ __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_eu(kNextSample ? RGRT_SHADE_WAVES : kAhead ? RGRT_SHADE_AHEAD_WAVES : RGRT_SHADE1_WAVES))) void k_shade(ShadeParams p, int cur, int ahead)
 {
-    const uint32_t count = p.st.counters[cur];
+    const QueueSpan queue(p.st, cur);
     const int lane = threadIdx.x & 63;
     const uint64_t ltMask = lane == 0 ? 0ull : ((~0ull) >> (64 - lane));
     const Ctx c{p, f3(p.ubo.lightDir[0], p.ubo.lightDir[1], p.ubo.lightDir[2]), p.ubo.maxRecursions, 0u,
                 ahead ? p.st.counters + kAheadCountWord + (1 - cur) : nullptr};
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for(uint32_t base = blockIdx.x * blockDim.x + (threadIdx.x & ~63u); base < count; base += stride)
-        shade_wave<kNextSample, kAhead>(p, c, cur, count, base, lane, ltMask);
+    const uint32_t waves = gridDim.x * (kShadeBlock / 64);
+    for(uint32_t k = blockIdx.x * (kShadeBlock / 64) + (threadIdx.x >> 6); k < queue.chunks; k += waves)
+        shade_wave<kNextSample, kAhead>(p, c, cur, queue, k, lane, ltMask);
 }
 
 // Scene of a batch that chunk k (64 queue entries) belongs to, from the
@@ -1154,7 +1154,7 @@ __device__ __forceinline__ void batch_chunk_prefix(const ShadeParams* ps, int nu
 {
     if(threadIdx.x < 64) {
         const int lane = threadIdx.x;
-        uint32_t v = lane < numScenes ? (ps[lane].st.counters[cur] + 63u) / 64u : 0u;
+        uint32_t v = lane < numScenes ? QueueSpan(ps[lane].st, cur).chunks : 0u;
         for(int off = 1; off < 64; off <<= 1) {
             const uint32_t u = __shfl_up(v, off);
             if(lane >= off) v += u;
@@ -1182,7 +1182,7 @@ __global__ __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_eu(kNe
         const ShadeParams& p = ps[s];
         const uint32_t first = s ? chunkEnd[s - 1] : 0u;
         const Ctx c{p, f3(p.ubo.lightDir[0], p.ubo.lightDir[1], p.ubo.lightDir[2]), p.ubo.maxRecursions, 0u, nullptr};
-        shade_wave<kNextSample, false>(p, c, cur, p.st.counters[cur], (k - first) * 64u, lane, ltMask);
+        shade_wave<kNextSample, false>(p, c, cur, QueueSpan(p.st, cur), k - first, lane, ltMask);
     }
 }
 
@@ -1199,7 +1199,8 @@ constexpr int kDrainSpill = 368; // see traverse.h: 16 + 368 >= 382
 template<bool kNextSample, bool kAhead, typename Stack>
 __device__ __forceinline__ void drain_scene(const ShadeParams& p, const TraceScene& sc, int cur, Stack& stack)
 {
-    const uint32_t count = p.st.counters[cur];
+    const QueueSpan queue(p.st, cur);
+    const uint32_t count = queue.count();
     const size_t n = p.st.npix;
     const float* __restrict__ rays = p.st.rays[cur];
     uint32_t* fetch = p.st.counters + 2 + cur;
@@ -1222,8 +1223,9 @@ __device__ __forceinline__ void drain_scene(const ShadeParams& p, const TraceSce
                 b = __shfl(b, 0);
                 if(b + (uint32_t)__popcll(idle) >= count) exhausted = true;
                 if(!active) {
-                    const uint32_t i = b + (uint32_t)__popcll(idle & ltMask);
+                    uint32_t i = b + (uint32_t)__popcll(idle & ltMask);
                     if(i < count) {
+                        if(i >= queue.front) i = queue.size - 1u - (i - queue.front);
                         pix = __float_as_uint(rays[8 * n + i]);
                         flags = __float_as_uint(rays[9 * n + i]);
                         r.ox = rays[0 * n + i];

@@ -49,3 +49,25 @@ def test_rays_ahead_change_no_image(passes, stochastic):
             assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("size", [(1024, 1024), (1025, 1024)])
+def test_frames_on_both_sides_of_the_sorted_queue_rule(size):
+    """Frames of up to 2^20 slots append every ray at the queue's front, larger
+    ones shadow rays there and others at its back: in one piece and in bands,
+    the images are those of the drain alone (which appends nothing)."""
+    print(f"[case] sorted queue {size}", flush=True)
+    setup = glass_scene(*size, 3)
+    setup.num_samples = 1
+    ctx, _ = gpu_context(setup)
+    try:
+        seen = []
+        for passes, bands in ((0, 1), (5, 1), (64, 1), (5, 3)):
+            ctx.set_tuning(wavefrontPasses=passes, frameBands=bands)
+            ctx.render(True)
+            seen.append((ctx.read_image(rgrt.IMAGE_FINAL), ctx.stats()["rays"]))
+        for image, rays in seen[1:]:
+            assert rays == seen[0][1]
+            assert np.array_equal(image, seen[0][0])
+    finally:
+        ctx.close()
