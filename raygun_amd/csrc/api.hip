@@ -12,6 +12,7 @@
 namespace rgrt {
 uint32_t trace_spill_words_per_thread();
 uint32_t trace_block_size();
+uint32_t trace_resident_blocks();
 void launch_trace_queue_impl(hipStream_t s, const TraceScene& sc, const WavefrontState& st, int cur, uint32_t gridBlocks,
                              int32_t* spill, uint32_t* hostSlot, bool ahead);
 void launch_trace_rays_impl(hipStream_t s, const TraceScene& sc, const rgrt_ray* rays, uint32_t n, uint32_t cullMask,
@@ -176,7 +177,10 @@ struct rgrt_ctx {
     // per band (the bands' launches run side by side).
     void apply_tuning()
     {
-        traceGrid = numCUs * tuning.traceBlocksPerCU;
+        // the traversal grid is persistent: blocks past what a CU holds would
+        // start on their share when the others are done (4K at 4 samples with
+        // six blocks per CU, five of them resident: 95.8 ms, clamped 86.0)
+        traceGrid = numCUs * std::min(tuning.traceBlocksPerCU, trace_resident_blocks());
         shadeGrid = numCUs * tuning.shadeBlocksPerCU;
         drainGrid = numCUs * tuning.drainBlocksPerCU;
         bands = std::max<uint32_t>(1u, std::min(tuning.frameBands, kMaxBands));
@@ -395,6 +399,7 @@ void free_images(rgrt_ctx* c)
     dev_free(s.rays[1]);
     dev_free(s.hits);
     dev_free(s.ahead);
+    dev_free(s.segs);
     dev_free(s.sampleAcc);
     dev_free(s.sampleLum2);
     c->slotCap = 0;
@@ -463,6 +468,7 @@ void alloc_images(rgrt_ctx* c, uint32_t w, uint32_t h)
     dev_alloc(s.rays[1], npix * kRayWords);
     dev_alloc(s.hits, npix * kHitWords);
     dev_alloc(s.ahead, ahead_words(npix));
+    dev_alloc(s.segs, kMaxBands * kSegmentBlock);
     dev_alloc(s.counters, 64);
     check(hipMemsetAsync(s.counters, 0, 64 * 4, c->stream));
     c->w = w;
@@ -612,6 +618,7 @@ void prepare_sample_groups(rgrt_ctx* c)
     s.npix = (uint32_t)slots;
     s.chunkFirst = 0;
     s.frameSlots = (uint32_t)slots;
+    s.segments = segments_for((uint32_t)slots);
     s.groups = g;
     s.numSamples = n;
 }
@@ -728,9 +735,14 @@ rgrt_status do_trace(rgrt_ctx* c)
     if(!drained && it == maxIters) {
         // all pixels must be done after the bound; check the last count
         check(hipStreamSynchronize(s));
-        uint32_t counts[kCounterBlock];
-        check(hipMemcpy(counts, c->st.counters, sizeof(counts), hipMemcpyDeviceToHost));
-        if(counts[cur] + counts[kQueueBackWord + cur]) return fail(c, RGRT_ERR_HIP, "rgrt_trace: ray queue did not drain within the recursion bound");
+        std::vector<uint32_t> counts(kSegmentBlock);
+        check(hipMemcpy(counts.data(), c->st.segs, kSegmentBlock * 4, hipMemcpyDeviceToHost));
+        uint32_t remaining = 0;
+        for(uint32_t q = 0; q < kMaxSegments; ++q) {
+            const uint32_t* n = &counts[(cur * kMaxSegments + q) * kSegmentWords];
+            remaining += n[0] + n[1];
+        }
+        if(remaining) return fail(c, RGRT_ERR_HIP, "rgrt_trace: ray queue did not drain within the recursion bound");
     }
     launch_finalize_samples(s, p);
     if(timing) check(hipEventRecord(c->evRtOnlyEnd, s));
@@ -800,6 +812,8 @@ WavefrontState band_state(const WavefrontState& st, uint32_t b, uint32_t bands)
     w.hits = st.hits + (size_t)kHitWords * q0;
     w.ahead = st.ahead + (size_t)kAheadWords * kAheadPerSlot * q0;
     w.counters = st.counters + (size_t)kCounterBlock * b;
+    w.segs = st.segs + (size_t)kSegmentBlock * b;
+    w.segments = segments_for(slots);
     return w;
 }
 
@@ -1780,6 +1794,7 @@ rgrt_status batch_frame_persistent(rgrt_batch* b, const rgrt_frame_desc* descs)
         uint32_t chain = 1;
         for(uint32_t i = 0; i < n; ++i) {
             ps[i] = shade_params(b->ctxs[i]);
+            ps[i].st.segments = 1; // the merged launches take a scene's queue in one piece
             scs[i] = b->ctxs[i]->scene();
             chain = std::max(chain, chain_iters(b->ctxs[i]));
         }

@@ -150,41 +150,133 @@ struct WavefrontState {
     float* rays[2] = {nullptr, nullptr}; // [kRayWords][npix]
     float* hits = nullptr;    // [kHitWords][npix]
     float* ahead = nullptr;   // [kAheadWords][kAheadPerSlot * npix]: rays traced ahead by the next pass
-    // [0..1] rays at the front of queue 0, 1, [2..3] fetch, [4..9] stats (u64 pairs), [10..11] rays ahead, [12]
-    // traversal errors, [13..14] rays at the back of queue 0, 1
-    uint32_t* counters = nullptr;
+    uint32_t segments = 1;        // strips of the queues (QueueSpan)
+    uint32_t* segs = nullptr;     // [2][kMaxSegments][kSegmentWords]: rays at the front and back of each strip
+    uint32_t* counters = nullptr; // [2..3] fetch, [4..9] stats (u64 pairs), [10..11] rays ahead, [12] traversal errors
     float* lum2 = nullptr;        // [npix]: sum of squared sample luminances (stochastic sampling)
 };
 
-constexpr int kQueueBackWord = 13;
-
-// Queue `cur` of a frame (or band): in frames of more than kSortedSlots slots
-// shadow rays fill it from the front and all others from the back, so a wave's
-// 64 entries are of one sort (shadow rays of neighbouring pixels run in
-// parallel, and their shading takes one path): 4K at 4 samples 94.2 -> 91.4
-// ms, 1080p over 2M triangles 8.62 -> 8.49. Smaller frames, whose passes wait
-// on their slowest rays, keep one end (split, 960x540 over 3,000 instances
-// measured 3.44 -> 3.47 ms, 640x360 0.456 -> 0.459). Work on it is cut into
-// 64-entry chunks, the front's then the back's.
+// A frame's queue is cut into `segments` strips of slots, each with its own part
+// of the queue and its own counters: a slot's rays stay in its strip. With
+// one counter for the whole queue the appends of a pass, one atomic per wave,
+// took 10-12 ns each whatever else the pass did (a first pass of 8.3M rays:
+// 1.55 ms of shading with the VALUs 9% busy). In strips, and with three quarters
+// of the traversal's chunks no longer fetched from a counter: 1080p at 4
+// samples with the denoiser 7.67 -> 4.90 ms, 4K at 4 samples 91.5 -> 86.0,
+// 1080p over 2M triangles 8.51 -> 8.12, 960x540 over 3,000 instances 3.45 ->
+// 3.24. A strip has at least 16384 slots (256 waves in the first pass): thinner
+// ones would only leave more chunks partly filled.
+//
+// Within a strip, in frames of more than kSortedSlots slots shadow rays fill
+// the queue from the front and all others from the back, so a wave's 64
+// entries are of one sort (shadow rays of neighbouring pixels run in parallel,
+// and their shading takes one path): 4K at 4 samples 94.2 -> 91.4 ms, 1080p
+// over 2M triangles 8.62 -> 8.49. Smaller frames, whose passes wait on their
+// slowest rays, keep one end (split, 960x540 over 3,000 instances measured
+// 3.44 -> 3.47 ms, 640x360 0.456 -> 0.459).
+//
+// Work on a queue is cut into 64-entry chunks: strip by strip, the front's
+// then the back's, so a chunk is of one strip.
+constexpr uint32_t kMaxSegments = 64;
+constexpr uint32_t kSegmentWords = 16; // a counter pair (front, back) on a 64-byte line of its own
+constexpr uint32_t kSegmentSlots = 1u << 14; // a strip has at least this many slots
 constexpr uint32_t kSortedSlots = 1u << 20;
+constexpr uint32_t kSegmentBlock = 2 * kMaxSegments * kSegmentWords; // counter words of a band's two queues
+
+__host__ __device__ inline uint32_t segments_for(uint32_t slots)
+{
+    const uint32_t n = slots / kSegmentSlots;
+    return n < 1u ? 1u : n > kMaxSegments ? kMaxSegments : n;
+}
+
+__device__ __forceinline__ uint32_t* segment_counts(const WavefrontState& st, int queue, uint32_t segment)
+{
+    return st.segs + ((uint32_t)queue * kMaxSegments + segment) * kSegmentWords;
+}
+// First queue position (and slot of the band) of a strip.
+__device__ __forceinline__ uint32_t segment_start(const WavefrontState& st, uint32_t segment)
+{
+    const uint32_t chunks = (st.npix + 63u) / 64u;
+    const uint32_t at = (uint32_t)((uint64_t)chunks * segment / st.segments) * 64u;
+    return at < st.npix ? at : st.npix;
+}
+
+// A strip's part of queue `queue`.
 struct QueueSpan {
-    uint32_t front, back, frontChunks, chunks, size;
-    __device__ __forceinline__ QueueSpan(const WavefrontState& st, int cur)
+    uint32_t front, back, frontChunks, chunks, start, end;
+    __device__ __forceinline__ QueueSpan(const WavefrontState& st, uint32_t segment, uint32_t f, uint32_t b)
+        : front(f), back(b), frontChunks((f + 63u) / 64u), chunks((f + 63u) / 64u + (b + 63u) / 64u),
+          start(segment_start(st, segment)), end(segment_start(st, segment + 1u))
     {
-        front = st.counters[cur];
-        back = st.counters[kQueueBackWord + cur];
-        frontChunks = (front + 63u) / 64u;
-        chunks = frontChunks + (back + 63u) / 64u;
-        size = st.npix;
+    }
+    __device__ __forceinline__ QueueSpan(const WavefrontState& st, int queue, uint32_t segment)
+        : QueueSpan(st, segment, segment_counts(st, queue, segment)[0], segment_counts(st, queue, segment)[1])
+    {
     }
     __device__ __forceinline__ uint32_t count() const { return front + back; }
-    // Queue position of a lane of chunk k; false past its end.
+    // Queue position of a lane of the strip's chunk k; false past its end.
     __device__ __forceinline__ bool entry(uint32_t k, uint32_t lane, uint32_t& i) const
     {
         const bool isBack = k >= frontChunks;
         const uint32_t j = (isBack ? k - frontChunks : k) * 64u + lane;
-        i = isBack ? size - 1u - j : j;
+        i = isBack ? end - 1u - j : start + j;
         return j < (isBack ? back : front);
+    }
+    // Queue position of the strip's j-th entry.
+    __device__ __forceinline__ uint32_t at(uint32_t j) const { return j < front ? start + j : end - 1u - (j - front); }
+};
+
+// All strips of a queue, in a block's LDS: inclusive prefixes over the strips
+// of their chunks and entries.
+struct QueueMap {
+    uint32_t chunkEnd[kMaxSegments], entryEnd[kMaxSegments];
+    uint32_t front[kMaxSegments], back[kMaxSegments];
+
+    // By the whole block (a barrier inside).
+    __device__ __forceinline__ void load(const WavefrontState& st, int queue)
+    {
+        if(threadIdx.x < 64u) {
+            const uint32_t lane = threadIdx.x;
+            uint32_t f = 0, b = 0;
+            if(lane < st.segments) {
+                f = segment_counts(st, queue, lane)[0];
+                b = segment_counts(st, queue, lane)[1];
+            }
+            uint32_t v = (f + 63u) / 64u + (b + 63u) / 64u, e = f + b;
+            for(int off = 1; off < 64; off <<= 1) {
+                const uint32_t v1 = __shfl_up(v, off), e1 = __shfl_up(e, off);
+                if((int)lane >= off) {
+                    v += v1;
+                    e += e1;
+                }
+            }
+            chunkEnd[lane] = v;
+            entryEnd[lane] = e;
+            front[lane] = f;
+            back[lane] = b;
+        }
+        __syncthreads();
+    }
+    __device__ __forceinline__ uint32_t chunks() const { return chunkEnd[kMaxSegments - 1]; }
+    __device__ __forceinline__ uint32_t count() const { return entryEnd[kMaxSegments - 1]; }
+    // Strip of chunk k (uniform over the wave); k becomes the chunk within it.
+    __device__ __forceinline__ uint32_t segment(uint32_t lane, uint32_t& k) const
+    {
+        const uint32_t s = (uint32_t)__builtin_amdgcn_readfirstlane(__popcll(__ballot(chunkEnd[lane] <= k)));
+        if(s) k -= chunkEnd[s - 1u];
+        return s;
+    }
+    __device__ __forceinline__ QueueSpan span(const WavefrontState& st, uint32_t segment) const
+    {
+        return QueueSpan(st, segment, front[segment], back[segment]);
+    }
+    // Queue position of entry i of all strips' (per lane).
+    __device__ __forceinline__ uint32_t at(const WavefrontState& st, uint32_t i) const
+    {
+        uint32_t s = 0;
+        for(uint32_t step = kMaxSegments / 2; step > 0; step /= 2)
+            if(entryEnd[s + step - 1u] <= i) s += step;
+        return span(st, s).at(s ? i - entryEnd[s - 1u] : i);
     }
 };
 

@@ -29,17 +29,20 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(RGR
     TraceScene sc, WavefrontState st, int cur, int32_t* __restrict__ spillBase, uint32_t* hostSlot)
 {
     __shared__ int32_t ldsStack[kLdsStack * kTraceBlock];
+    __shared__ QueueMap queue;
     uint32_t* counters = st.counters;
     const float* __restrict__ rays = st.rays[cur];
     float* __restrict__ hits = st.hits;
     const size_t npix = st.npix;
     const size_t aheadCap = npix * kAheadPerSlot;
-    const QueueSpan queue(st, cur);
+    queue.load(st, cur);
     const uint32_t ahead = kAhead ? (uint32_t)min((size_t)counters[kAheadCountWord + cur], aheadCap) : 0u;
+    if(blockIdx.x == 0 && threadIdx.x < kMaxSegments) { // the output queue of the shading pass that follows
+        segment_counts(st, 1 - cur, threadIdx.x)[0] = 0;
+        segment_counts(st, 1 - cur, threadIdx.x)[1] = 0;
+    }
     if(blockIdx.x == 0 && threadIdx.x == 0) {
         *hostSlot = queue.count() + ahead; // host-visible: lets the host stop once the queues drain
-        counters[1 - cur] = 0;             // the output queues of the shading pass that follows
-        counters[kQueueBackWord + (1 - cur)] = 0;
         counters[kAheadCountWord + (1 - cur)] = 0;
         counters[2 + (1 - cur)] = 0; // the fetch counter of the next traversal pass
         // ray statistics (64-bit) at counters[4..5]
@@ -51,16 +54,29 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(RGR
     TraversalStack<kLdsStack, kTraceBlock, kSpill> stack{ldsStack, spillBase + (size_t)gtid * kSpill, (int)threadIdx.x, boxRay};
     uint32_t* fetch = counters + 2 + cur;
     // The work is cut into chunks of 64 rays: the queue's, then those of the
-    // rays queued ahead. Wave w first takes chunk w; chunks beyond the grid's
-    // static share are fetched from a counter, so a pass with fewer rays than
-    // the grid has lanes does no atomics at all.
+    // rays queued ahead. Wave w first takes chunks w, w + waves, ... (three
+    // quarters of its share, at least one); the rest are fetched from a counter,
+    // which evens out the waves. A pass with fewer rays than the grid has lanes
+    // does no atomics at all.
     const uint32_t wavesInGrid = gridDim.x * (kTraceBlock / 64);
-    const uint32_t chunks = queue.chunks + (ahead + 63u) / 64u;
+    const uint32_t mainChunks = queue.chunks();
+    const uint32_t chunks = mainChunks + (ahead + 63u) / 64u;
+    const uint32_t rounds = max(1u, chunks * 3u / (wavesInGrid * 4u));
     uint32_t k = blockIdx.x * (kTraceBlock / 64) + (threadIdx.x >> 6);
-    while(k < chunks) {
-        const bool isAhead = kAhead && k >= queue.chunks;
-        uint32_t i = isAhead ? (k - queue.chunks) * 64u + lane : 0u;
-        if(isAhead ? i < ahead : queue.entry(k, lane, i)) {
+    for(uint32_t round = 1; k < chunks; ++round) {
+        const bool isAhead = kAhead && k >= mainChunks;
+        uint32_t i;
+        bool mine;
+        if(isAhead) {
+            i = (k - mainChunks) * 64u + lane;
+            mine = i < ahead;
+        }
+        else {
+            uint32_t within = k;
+            const uint32_t s = queue.segment((uint32_t)lane, within);
+            mine = queue.span(st, s).entry(within, (uint32_t)lane, i);
+        }
+        if(mine) {
             RayIn r;
             uint32_t mask, slot = 0;
             if(isAhead) {
@@ -102,9 +118,13 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(RGR
                 hits[4 * npix + i] = __uint_as_float(h.prim);
             }
         }
-        if(chunks <= wavesInGrid) break; // no rays beyond the static share
+        if(chunks <= wavesInGrid) break; // no rays beyond the first chunks
+        if(round < rounds) {
+            k += wavesInGrid;
+            continue;
+        }
         uint32_t b = 0;
-        if(lane == 0) b = wavesInGrid + atomicAdd(fetch, 1u);
+        if(lane == 0) b = rounds * wavesInGrid + atomicAdd(fetch, 1u);
         k = __shfl(b, 0);
     }
 }
@@ -126,7 +146,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(RGR
     if(threadIdx.x < 64) {
         uint32_t count = 0, v = 0;
         if(lane < numScenes) {
-            const QueueSpan queue(ps[lane].st, cur);
+            const QueueSpan queue(ps[lane].st, cur, 0u);
             count = queue.count();
             v = queue.chunks;
         }
@@ -138,8 +158,8 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(RGR
         if(blockIdx.x == 0) {
             if(lane < numScenes) {
                 uint32_t* counters = ps[lane].st.counters;
-                counters[1 - cur] = 0;       // the output queue of the shading pass that follows
-                counters[kQueueBackWord + (1 - cur)] = 0;
+                segment_counts(ps[lane].st, 1 - cur, 0u)[0] = 0; // the output queue of the shading pass that follows
+                segment_counts(ps[lane].st, 1 - cur, 0u)[1] = 0;
                 counters[2 + (1 - cur)] = 0; // the fetch counter of the drain
                 atomicAdd(reinterpret_cast<unsigned long long*>(counters + 4), (unsigned long long)count);
             }
@@ -159,7 +179,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(RGR
         const uint32_t first = s ? chunkEnd[s - 1] : 0u;
         const WavefrontState& st = ps[s].st;
         uint32_t i;
-        if(QueueSpan(st, cur).entry(k - first, (uint32_t)lane, i)) {
+        if(QueueSpan(st, cur, 0u).entry(k - first, (uint32_t)lane, i)) {
             const size_t npix = st.npix;
             const float* __restrict__ rays = st.rays[cur];
             float* __restrict__ hits = st.hits;
@@ -224,6 +244,13 @@ __global__ void k_hit_custom_index(rgrt_hit* hits, uint32_t n, const InstanceSha
 
 uint32_t trace_spill_words_per_thread() { return kSpill; }
 uint32_t trace_block_size() { return kTraceBlock; }
+// Blocks of the traversal pass a CU holds.
+uint32_t trace_resident_blocks()
+{
+    int n = 0;
+    check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_trace_queue<false>, kTraceBlock, 0));
+    return (uint32_t)std::max(1, n);
+}
 
 void launch_trace_queue_impl(hipStream_t s, const TraceScene& sc, const WavefrontState& st, int cur, uint32_t gridBlocks,
                              int32_t* spill, uint32_t* hostSlot, bool ahead)

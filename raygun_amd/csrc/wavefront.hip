@@ -52,12 +52,12 @@ constexpr int kShadeBlock = 256;
 #ifndef RGRT_DRAIN_WAVES
 #define RGRT_DRAIN_WAVES 1
 #endif
-// The shading variant for one sample per slot fits in 128 VGPRs (4 waves);
-// compiled for 5 waves it spills 29 VGPRs and is slightly faster beside
-// other frames' traversal (config 2 at 1080p, four frames in flight:
-// 5.36 against 5.40-5.43 ms per frame).
+// The shading variant for one sample per slot fits in 128 VGPRs (4 waves). At 5
+// waves it spills 31, which is slower since its appends no longer wait on one
+// counter: 4K at 4 samples 86.0 against 83.6 ms, 1080p at 4 samples with the
+// denoiser 4.90 against 4.64 ms per frame.
 #ifndef RGRT_SHADE1_WAVES
-#define RGRT_SHADE1_WAVES 5
+#define RGRT_SHADE1_WAVES 4
 #endif
 // The drain variant for one sample per slot (no next-sample start) fits in
 // 143 VGPRs (3 waves); compiled for 4 waves it spills 12 VGPRs and runs
@@ -870,12 +870,15 @@ __device__ __forceinline__ void write_ray(float* rays, size_t n, uint32_t slot, 
 // Primary ray of the band's slot `q`, at position q of the band's queue 0.
 __device__ __forceinline__ void raygen_slot(const ShadeParams& p, uint32_t q)
 {
+    if(q < kMaxSegments) { // queue 0 holds every slot's primary ray
+        const bool used = q < p.st.segments;
+        segment_counts(p.st, 0, q)[0] = used ? segment_start(p.st, q + 1u) - segment_start(p.st, q) : 0u;
+        segment_counts(p.st, 0, q)[1] = 0;
+        segment_counts(p.st, 1, q)[0] = 0;
+        segment_counts(p.st, 1, q)[1] = 0;
+    }
     if(q == 0) {
         uint32_t* c = p.st.counters;
-        c[0] = p.st.npix; // queue 0 holds every slot's primary ray
-        c[1] = 0;
-        c[kQueueBackWord] = 0;
-        c[kQueueBackWord + 1] = 0;
         c[2] = 0;
         c[3] = 0;
         for(int k = 4; k < 12; ++k) c[k] = 0; // ray / sky / zero-dir counters (u64), rays ahead
@@ -1088,12 +1091,12 @@ __device__ __forceinline__ HitRec load_hit(const float* hits, size_t n, uint32_t
     return h;
 }
 
-// Shades chunk k of queue `cur` (one wave, one lane per entry), appending the
-// emitted rays to an end of the other queue (QueueSpan), one atomic instruction
-// per wave.
+// Shades chunk k of a strip of queue `cur` (one wave, one lane per entry),
+// appending the emitted rays to the ends of the strip's part of the other
+// queue (QueueSpan), one atomic instruction per wave.
 template<bool kNextSample, bool kAhead>
-__device__ __forceinline__ void shade_wave(const ShadeParams& p, const Ctx& c, int cur, const QueueSpan& queue, uint32_t k, int lane,
-                                           uint64_t ltMask)
+__device__ __forceinline__ void shade_wave(const ShadeParams& p, const Ctx& c, int cur, const QueueSpan& queue, uint32_t segment, uint32_t k,
+                                           int lane, uint64_t ltMask)
 {
     const size_t n = p.st.npix;
     const float* __restrict__ rays = p.st.rays[cur];
@@ -1118,9 +1121,9 @@ __device__ __forceinline__ void shade_wave(const ShadeParams& p, const Ctx& c, i
     if(toFront | toBack) {
         uint32_t base = 0;
         if(lane < 2)
-            base = atomicAdd(p.st.counters + (lane ? kQueueBackWord : 0) + (1 - cur), (uint32_t)__popcll(lane ? toBack : toFront));
+            base = atomicAdd(segment_counts(p.st, 1 - cur, segment) + lane, (uint32_t)__popcll(lane ? toBack : toFront));
         const uint32_t f0 = (uint32_t)__builtin_amdgcn_readlane((int)base, 0), b0 = (uint32_t)__builtin_amdgcn_readlane((int)base, 1);
-        const uint32_t at = front ? f0 + (uint32_t)__popcll(toFront & ltMask) : (uint32_t)n - 1u - (b0 + (uint32_t)__popcll(toBack & ltMask));
+        const uint32_t at = front ? queue.start + f0 + (uint32_t)__popcll(toFront & ltMask) : queue.end - 1u - (b0 + (uint32_t)__popcll(toBack & ltMask));
         if(emit) write_ray(outRays, n, at, out, pix, (out.mask << kMaskShift) | out.miss1);
     }
 }
@@ -1130,14 +1133,19 @@ __device__ __forceinline__ void shade_wave(const ShadeParams& p, const Ctx& c, i
 template<bool kNextSample, bool kAhead>
 __global__ __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_eu(kNextSample ? RGRT_SHADE_WAVES : kAhead ? RGRT_SHADE_AHEAD_WAVES : RGRT_SHADE1_WAVES))) void k_shade(ShadeParams p, int cur, int ahead)
 {
-    const QueueSpan queue(p.st, cur);
+    __shared__ QueueMap queue;
+    queue.load(p.st, cur);
+    const uint32_t chunks = queue.chunks();
     const int lane = threadIdx.x & 63;
     const uint64_t ltMask = lane == 0 ? 0ull : ((~0ull) >> (64 - lane));
     const Ctx c{p, f3(p.ubo.lightDir[0], p.ubo.lightDir[1], p.ubo.lightDir[2]), p.ubo.maxRecursions, 0u,
                 ahead ? p.st.counters + kAheadCountWord + (1 - cur) : nullptr};
     const uint32_t waves = gridDim.x * (kShadeBlock / 64);
-    for(uint32_t k = blockIdx.x * (kShadeBlock / 64) + (threadIdx.x >> 6); k < queue.chunks; k += waves)
-        shade_wave<kNextSample, kAhead>(p, c, cur, queue, k, lane, ltMask);
+    for(uint32_t k = blockIdx.x * (kShadeBlock / 64) + (threadIdx.x >> 6); k < chunks; k += waves) {
+        uint32_t within = k;
+        const uint32_t s = queue.segment((uint32_t)lane, within);
+        shade_wave<kNextSample, kAhead>(p, c, cur, queue.span(p.st, s), s, within, lane, ltMask);
+    }
 }
 
 // Scene of a batch that chunk k (64 queue entries) belongs to, from the
@@ -1154,7 +1162,7 @@ __device__ __forceinline__ void batch_chunk_prefix(const ShadeParams* ps, int nu
 {
     if(threadIdx.x < 64) {
         const int lane = threadIdx.x;
-        uint32_t v = lane < numScenes ? QueueSpan(ps[lane].st, cur).chunks : 0u;
+        uint32_t v = lane < numScenes ? QueueSpan(ps[lane].st, cur, 0u).chunks : 0u;
         for(int off = 1; off < 64; off <<= 1) {
             const uint32_t u = __shfl_up(v, off);
             if(lane >= off) v += u;
@@ -1182,7 +1190,7 @@ __global__ __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_eu(kNe
         const ShadeParams& p = ps[s];
         const uint32_t first = s ? chunkEnd[s - 1] : 0u;
         const Ctx c{p, f3(p.ubo.lightDir[0], p.ubo.lightDir[1], p.ubo.lightDir[2]), p.ubo.maxRecursions, 0u, nullptr};
-        shade_wave<kNextSample, false>(p, c, cur, QueueSpan(p.st, cur), k - first, lane, ltMask);
+        shade_wave<kNextSample, false>(p, c, cur, QueueSpan(p.st, cur, 0u), 0u, k - first, lane, ltMask);
     }
 }
 
@@ -1190,16 +1198,18 @@ constexpr int kDrainBlock = 256;
 constexpr int kDrainLdsStack = 16;
 constexpr int kDrainSpill = 368; // see traverse.h: 16 + 368 >= 382
 
+__device__ __forceinline__ uint32_t queue_at(const WavefrontState& st, const QueueMap& q, uint32_t i) { return q.at(st, i); }
+__device__ __forceinline__ uint32_t queue_at(const WavefrontState&, const QueueSpan& q, uint32_t i) { return q.at(i); }
+
 // Drain: finishes every pixel still in flight after the wavefront passes.
 // Each lane takes a queued ray, traces and shades it, and keeps tracing that
 // pixel's next rays itself until the pixel is done; idle lanes refill from
 // the queue (one atomic per wave, a ballot to hand out the entries). The
 // recursion tail thus costs the longest remaining chain of one pixel rather
 // than one launch per recursion step.
-template<bool kNextSample, bool kAhead, typename Stack>
-__device__ __forceinline__ void drain_scene(const ShadeParams& p, const TraceScene& sc, int cur, Stack& stack)
+template<bool kNextSample, bool kAhead, typename Queue, typename Stack>
+__device__ __forceinline__ void drain_scene(const ShadeParams& p, const TraceScene& sc, int cur, const Queue& queue, Stack& stack)
 {
-    const QueueSpan queue(p.st, cur);
     const uint32_t count = queue.count();
     const size_t n = p.st.npix;
     const float* __restrict__ rays = p.st.rays[cur];
@@ -1225,7 +1235,7 @@ __device__ __forceinline__ void drain_scene(const ShadeParams& p, const TraceSce
                 if(!active) {
                     uint32_t i = b + (uint32_t)__popcll(idle & ltMask);
                     if(i < count) {
-                        if(i >= queue.front) i = queue.size - 1u - (i - queue.front);
+                        i = queue_at(p.st, queue, i);
                         pix = __float_as_uint(rays[8 * n + i]);
                         flags = __float_as_uint(rays[9 * n + i]);
                         r.ox = rays[0 * n + i];
@@ -1278,7 +1288,9 @@ __global__ __launch_bounds__(kDrainBlock) __attribute__((amdgpu_waves_per_eu(kNe
     __shared__ float boxRay[kBoxRayWords * kDrainBlock];
     TraversalStack<kDrainLdsStack, kDrainBlock, kDrainSpill> stack{ldsStack, spillBase + (size_t)gtid * kDrainSpill,
                                                                    (int)threadIdx.x, boxRay};
-    drain_scene<kNextSample, kAhead>(p, sc, cur, stack);
+    __shared__ QueueMap queue;
+    queue.load(p.st, cur);
+    drain_scene<kNextSample, kAhead>(p, sc, cur, queue, stack);
 }
 
 // Drain of a whole batch: every wave drains the scenes in order, moving to
@@ -1297,7 +1309,7 @@ __global__ __launch_bounds__(kDrainBlock) __attribute__((amdgpu_waves_per_eu(kNe
                                                                    (int)threadIdx.x, boxRay};
     for(int s = 0; s < numScenes; ++s) {
         const TraceScene sc = scs[s];
-        drain_scene<kNextSample, false>(ps[s], sc, cur, stack);
+        drain_scene<kNextSample, false>(ps[s], sc, cur, QueueSpan(ps[s].st, cur, 0u), stack);
     }
 }
 

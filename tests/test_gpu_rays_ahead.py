@@ -51,12 +51,13 @@ def test_rays_ahead_change_no_image(passes, stochastic):
         ctx.close()
 
 
-@pytest.mark.parametrize("size", [(1024, 1024), (1025, 1024)])
-def test_frames_on_both_sides_of_the_sorted_queue_rule(size):
-    """Frames of up to 2^20 slots append every ray at the queue's front, larger
-    ones shadow rays there and others at its back: in one piece and in bands,
-    the images are those of the drain alone (which appends nothing)."""
-    print(f"[case] sorted queue {size}", flush=True)
+@pytest.mark.parametrize("size", [(9, 7), (256, 127), (256, 128), (1024, 1024), (1025, 1024)])
+def test_frames_on_both_sides_of_the_queue_rules(size):
+    """A frame's queue is in strips of at least 2^14 slots (at most 64), and above
+    2^20 slots shadow rays fill a strip from the front and others from the back:
+    in one piece and in bands, the images are those of the drain alone (which
+    appends nothing)."""
+    print(f"[case] queue rules {size}", flush=True)
     setup = glass_scene(*size, 3)
     setup.num_samples = 1
     ctx, _ = gpu_context(setup)
