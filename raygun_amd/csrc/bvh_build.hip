@@ -138,29 +138,41 @@ __global__ void k_scene_box_init(uint32_t* sb)
     else if(threadIdx.x < 6) sb[threadIdx.x] = float_to_ordered(-INFINITY);
 }
 
-__global__ void k_scene_box(const float4* __restrict__ boxLo, const float4* __restrict__ boxHi, uint32_t n, uint32_t* sb)
+// Few, large blocks: every block ends in six atomics on one cache line, which
+// take some 12 ns each whichever block they come from (1024 blocks of 256
+// threads: 40 us for 1M boxes, the reads alone 6).
+constexpr int kSceneBoxThreads = 1024;
+constexpr uint32_t kSceneBoxBlocks = 64;
+
+__global__ __launch_bounds__(kSceneBoxThreads) void k_scene_box(const float4* __restrict__ boxLo, const float4* __restrict__ boxHi,
+                                                                uint32_t n, uint32_t* sb)
 {
-    __shared__ uint32_t red[6];
-    if(threadIdx.x < 3) red[threadIdx.x] = float_to_ordered(INFINITY);
-    else if(threadIdx.x < 6) red[threadIdx.x] = float_to_ordered(-INFINITY);
-    __syncthreads();
-    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for(uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    __shared__ float red[6][kSceneBoxThreads / 64];
+    float v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    for(uint32_t i = blockIdx.x * kSceneBoxThreads + threadIdx.x; i < n; i += gridDim.x * kSceneBoxThreads) {
         const float4 a = boxLo[i], b = boxHi[i];
-        lo[0] = fminf(lo[0], a.x);
-        lo[1] = fminf(lo[1], a.y);
-        lo[2] = fminf(lo[2], a.z);
-        hi[0] = fmaxf(hi[0], b.x);
-        hi[1] = fmaxf(hi[1], b.y);
-        hi[2] = fmaxf(hi[2], b.z);
+        v[0] = fminf(v[0], a.x);
+        v[1] = fminf(v[1], a.y);
+        v[2] = fminf(v[2], a.z);
+        v[3] = fmaxf(v[3], b.x);
+        v[4] = fmaxf(v[4], b.y);
+        v[5] = fmaxf(v[5], b.z);
     }
-    for(int c = 0; c < 3; ++c) {
-        atomicMin(&red[c], float_to_ordered(lo[c]));
-        atomicMax(&red[3 + c], float_to_ordered(hi[c]));
+    for(int c = 0; c < 6; ++c) {
+        for(int off = 32; off > 0; off >>= 1) {
+            const float o = __shfl_xor(v[c], off);
+            v[c] = c < 3 ? fminf(v[c], o) : fmaxf(v[c], o);
+        }
+        if((threadIdx.x & 63) == 0) red[c][threadIdx.x >> 6] = v[c];
     }
     __syncthreads();
-    if(threadIdx.x < 3) atomicMin(&sb[threadIdx.x], red[threadIdx.x]);
-    else if(threadIdx.x < 6) atomicMax(&sb[threadIdx.x], red[threadIdx.x]);
+    if(threadIdx.x < 6) {
+        const int c = (int)threadIdx.x;
+        float r = red[c][0];
+        for(int w = 1; w < kSceneBoxThreads / 64; ++w) r = c < 3 ? fminf(r, red[c][w]) : fmaxf(r, red[c][w]);
+        if(c < 3) atomicMin(&sb[c], float_to_ordered(r));
+        else atomicMax(&sb[c], float_to_ordered(r));
+    }
 }
 
 // Morton code of a box centroid in the scene box sb (order-preserving integer encodings).
@@ -278,6 +290,35 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_apply(uint32_t* __restric
         if(i < e) hist[i] = carry + before + incl - c;
         carry += all;
         __syncthreads();
+    }
+}
+
+// The same over a short histogram in one workgroup, in place of the three
+// launches above (some 3 us each whatever their work).
+constexpr int kScanSmallThreads = 1024;
+constexpr uint32_t kScanSmallMax = 32768;
+
+__global__ __launch_bounds__(kScanSmallThreads) void k_scan_small(uint32_t* __restrict__ hist, uint32_t total)
+{
+    __shared__ uint32_t waveTot[kScanSmallThreads / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t per = (total + kScanSmallThreads - 1) / kScanSmallThreads;
+    const uint32_t b = min(total, threadIdx.x * per), e = min(total, b + per);
+    uint32_t sum = 0;
+    for(uint32_t i = b; i < e; ++i) sum += hist[i];
+    uint32_t incl = sum;
+    for(int off = 1; off < 64; off <<= 1) {
+        const uint32_t t = __shfl_up(incl, off);
+        if(lane >= off) incl += t;
+    }
+    if(lane == 63) waveTot[wave] = incl;
+    __syncthreads();
+    uint32_t at = incl - sum;
+    for(int w = 0; w < wave; ++w) at += waveTot[w];
+    for(uint32_t i = b; i < e; ++i) {
+        const uint32_t c = hist[i];
+        hist[i] = at;
+        at += c;
     }
 }
 
@@ -859,6 +900,165 @@ __global__ __launch_bounds__(kCollapseThreads) void k_collapse_numbered(const No
     if(tid == 0) *numWide = (uint32_t)base;
 }
 
+// The numbering of larger trees, in parallel. The wide nodes of one level cover
+// disjoint leaf ranges from left to right in breadth-first order, and a binary
+// node's index lies in its own range, so that order is the order of binary
+// indices: the numbering is a stable sort of the binary nodes that root a wide
+// node by their wide level (one pass of the radix sort, in index order). The
+// levels come from the top: one workgroup walks the nodes of more than
+// kSubtree leaves and lists the smaller subtrees hanging off them, then a wave
+// takes each of those.
+constexpr int kSubtree = 1024;
+constexpr uint32_t kNoWideNode = 255u; // sort digit of a binary node inside another's wide node
+constexpr int kDepthTopThreads = 1024;
+constexpr int kDepthSubThreads = 256;
+constexpr int kDepthSubBlocks = 512;
+constexpr int kSubFrontier = kSubtree / 2; // disjoint internal nodes, two leaves each at least
+
+__global__ void k_level_init(uint32_t* __restrict__ level, uint32_t* __restrict__ index, int numInternal)
+{
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if(r >= numInternal) return;
+    level[r] = kNoWideNode;
+    index[r] = (uint32_t)r;
+}
+
+__device__ __forceinline__ u32x4 candidate_children(const Node4* cand, int r)
+{
+    return ld_global16(reinterpret_cast<const u32x4*>(cand + r) + 6);
+}
+
+__global__ __launch_bounds__(kDepthTopThreads) void k_wide_levels_top(const Node4* __restrict__ cand,
+                                                                      const uint2* __restrict__ range, int numInternal,
+                                                                      uint32_t* level, uint32_t* frontA, uint32_t* frontB,
+                                                                      uint2* __restrict__ subtrees, uint32_t* numSubtrees)
+{
+    __shared__ uint32_t nextCount, subCount;
+    if(threadIdx.x == 0) {
+        subCount = 0;
+        frontA[0] = 0;
+        if(numInternal < kSubtree) { // the whole tree is one
+            subtrees[0] = make_uint2(0u, 0u);
+            subCount = 1;
+        }
+    }
+    __syncthreads();
+    uint32_t count = numInternal < kSubtree ? 0u : 1u;
+    for(uint32_t d = 0; d < 128u && count > 0u; ++d) {
+        if(threadIdx.x == 0) nextCount = 0;
+        __threadfence_block();
+        __syncthreads();
+        for(uint32_t k = threadIdx.x; k < count; k += kDepthTopThreads) {
+            const uint32_t r = frontA[k];
+            if(r >= (uint32_t)numInternal) continue;
+            level[r] = d;
+            const u32x4 ch = candidate_children(cand, (int)r);
+            const uint32_t c[4] = {ch.x, ch.y, ch.z, ch.w};
+#pragma unroll
+            for(int q = 0; q < 4; ++q) {
+                if((int)c[q] < 0 || c[q] >= (uint32_t)numInternal) continue;
+                const uint2 leaves = range[c[q]];
+                if(leaves.y - leaves.x >= (uint32_t)kSubtree) frontB[atomicAdd(&nextCount, 1u)] = c[q];
+                else subtrees[atomicAdd(&subCount, 1u)] = make_uint2(c[q], d + 1u);
+            }
+        }
+        __threadfence_block();
+        __syncthreads();
+        count = nextCount;
+        uint32_t* t = frontA;
+        frontA = frontB;
+        frontB = t;
+        __syncthreads();
+    }
+    if(threadIdx.x == 0) *numSubtrees = subCount;
+}
+
+__global__ __launch_bounds__(kDepthSubThreads) void k_wide_levels_sub(const Node4* __restrict__ cand, int numInternal,
+                                                                      uint32_t* __restrict__ level,
+                                                                      const uint2* __restrict__ subtrees,
+                                                                      const uint32_t* __restrict__ numSubtrees)
+{
+    constexpr int kWavesPerBlock = kDepthSubThreads / 64;
+    __shared__ uint32_t fronts[kWavesPerBlock][2][kSubFrontier];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint64_t ltMask = lane == 0 ? 0ull : ((~0ull) >> (64 - lane));
+    const uint32_t total = *numSubtrees;
+    for(uint32_t t = blockIdx.x * kWavesPerBlock + wave; t < total; t += gridDim.x * kWavesPerBlock) {
+        const uint2 root = subtrees[t];
+        uint32_t* front = fronts[wave][0];
+        uint32_t* next = fronts[wave][1];
+        if(lane == 0) front[0] = root.x;
+        uint32_t count = 1;
+        for(uint32_t d = root.y; d < 128u && count > 0u; ++d) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            uint32_t nextCount = 0;
+            for(uint32_t k = 0; k < count; k += 64u) {
+                const uint32_t i = k + (uint32_t)lane;
+                uint32_t c[4] = {0x80000000u, 0x80000000u, 0x80000000u, 0x80000000u};
+                if(i < count) {
+                    const uint32_t r = front[i];
+                    if(r < (uint32_t)numInternal) {
+                        level[r] = d;
+                        const u32x4 ch = candidate_children(cand, (int)r);
+                        c[0] = ch.x;
+                        c[1] = ch.y;
+                        c[2] = ch.z;
+                        c[3] = ch.w;
+                    }
+                }
+#pragma unroll
+                for(int q = 0; q < 4; ++q) {
+                    const bool in = (int)c[q] >= 0;
+                    const uint64_t m = __ballot(in);
+                    const uint32_t at = nextCount + (uint32_t)__popcll(m & ltMask);
+                    if(in && at < (uint32_t)kSubFrontier) next[at] = c[q];
+                    nextCount += (uint32_t)__popcll(m);
+                }
+            }
+            count = min(nextCount, (uint32_t)kSubFrontier);
+            uint32_t* x = front;
+            front = next;
+            next = x;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// The wide number of every binary node that roots one, and their count (where
+// the sort put the first node of digit kNoWideNode).
+__global__ void k_wide_numbers(const uint32_t* __restrict__ order, const uint32_t* __restrict__ hist, uint32_t numBlocks,
+                               int numInternal, uint32_t* __restrict__ number, uint32_t* numWide)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t nw = min(hist[kNoWideNode * numBlocks], (uint32_t)numInternal);
+    if(i == 0) *numWide = nw;
+    if(i < nw) number[order[i]] = i;
+}
+
+// Every wide node from its candidate, in parallel: 16-byte piece q of wide node
+// i comes from candidate order[i], the child refs (piece 6) renumbered.
+__global__ void k_wide_nodes(const Node4* __restrict__ cand, const uint32_t* __restrict__ order,
+                             const uint32_t* __restrict__ number, const uint32_t* __restrict__ numWide, int capacity,
+                             Node4* __restrict__ out)
+{
+    const long piece = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long i = piece >> 3;
+    const int q = (int)(piece & 7);
+    if(i >= min((long)*numWide, (long)capacity)) return;
+    const uint32_t r = order[i];
+    if(r >= (uint32_t)capacity) return;
+    u32x4 v = ld_global16(reinterpret_cast<const u32x4*>(cand + r) + q);
+    if(q == 6) {
+        v.x = v.x < (uint32_t)capacity ? number[v.x] : v.x;
+        v.y = v.y < (uint32_t)capacity ? number[v.y] : v.y;
+        v.z = v.z < (uint32_t)capacity ? number[v.z] : v.z;
+        v.w = v.w < (uint32_t)capacity ? number[v.w] : v.w;
+    }
+    reinterpret_cast<u32x4*>(out + i)[q] = v;
+}
+
 // The rest of every wide node (the child boxes and the padding, seven of its
 // eight 16-byte pieces) from its candidate, in parallel: piece q of wide node
 // i comes from candidate order[i].
@@ -1333,6 +1533,27 @@ void LbvhBuilder::release()
     capacity = 0;
 }
 
+namespace {
+// One stable pass of the radix sort; `partial` holds kScanBlocks words of
+// scratch (used only when the histogram is long, so when n is far above that).
+void sort_pass(hipStream_t s, const uint32_t* kin, const uint32_t* vin, uint32_t* kout, uint32_t* vout, uint32_t n, int shift,
+               uint32_t* hist, uint32_t* partial)
+{
+    const uint32_t nb = blocks_for(n, kSortTile);
+    const uint32_t total = 256u * nb;
+    k_sort_hist<<<nb, kSortThreads, 0, s>>>(kin, n, shift, hist, nb);
+    if(total <= kScanSmallMax) {
+        k_scan_small<<<1, kScanSmallThreads, 0, s>>>(hist, total);
+    }
+    else {
+        k_scan_reduce<<<kScanBlocks, kScanThreads, 0, s>>>(hist, total, partial);
+        k_scan_partials<<<1, kScanThreads, 0, s>>>(partial);
+        k_scan_apply<<<kScanBlocks, kScanThreads, 0, s>>>(hist, total, partial);
+    }
+    k_sort_scatter<<<nb, kSortThreads, 0, s>>>(kin, vin, kout, vout, n, shift, hist, nb);
+}
+} // namespace
+
 // Builds the hierarchy over boxLo/boxHi[0..n) (already filled). Writes
 // max(n-1,1) nodes, the Morton-ordered primitive ids and the root box.
 void LbvhBuilder::build(hipStream_t s, uint32_t n, Node* nodes, uint32_t* leafPrimOut, float4* rootBox)
@@ -1343,18 +1564,11 @@ void LbvhBuilder::build(hipStream_t s, uint32_t n, Node* nodes, uint32_t* leafPr
         return;
     }
     k_scene_box_init<<<1, 64, 0, s>>>(sceneBox);
-    const uint32_t sbBlocks = std::min<uint32_t>(blocks_for(n, 256), 1024);
-    k_scene_box<<<sbBlocks, 256, 0, s>>>(boxLo, boxHi, n, sceneBox);
+    k_scene_box<<<std::min(blocks_for(n, kSceneBoxThreads), kSceneBoxBlocks), kSceneBoxThreads, 0, s>>>(boxLo, boxHi, n, sceneBox);
     k_morton<<<blocks_for(n, 256), 256, 0, s>>>(boxLo, boxHi, n, sceneBox, keysA, valsA);
-    const uint32_t nb = blocks_for(n, kSortTile);
     uint32_t *kin = keysA, *vin = valsA, *kout = keysB, *vout = valsB;
     for(int shift = 0; shift < 32; shift += 8) {
-        k_sort_hist<<<nb, kSortThreads, 0, s>>>(kin, n, shift, hist, nb);
-        // counters[] is free until the refit: it holds the segment totals
-        k_scan_reduce<<<kScanBlocks, kScanThreads, 0, s>>>(hist, 256u * nb, counters);
-        k_scan_partials<<<1, kScanThreads, 0, s>>>(counters);
-        k_scan_apply<<<kScanBlocks, kScanThreads, 0, s>>>(hist, 256u * nb, counters);
-        k_sort_scatter<<<nb, kSortThreads, 0, s>>>(kin, vin, kout, vout, n, shift, hist, nb);
+        sort_pass(s, kin, vin, kout, vout, n, shift, hist, counters); // counters[] is free until the refit
         std::swap(kin, kout);
         std::swap(vin, vout);
     }
@@ -1398,12 +1612,36 @@ __global__ void k_leaf_parents(const Node* __restrict__ nodes, uint32_t numInter
 }
 } // namespace
 
+// Up to this many leaves the one-workgroup numbering's single launch costs less
+// than the sort's eight: a rebuild with contact rays takes 130 us for 32k
+// triangles against 151 (submitted back to back; alone 349 against 335), at 64k
+// both take 150, for 1M triangles it is 1138 against 600 us (alone 2303
+// against 971; the numbering itself 1348 against 140).
+constexpr uint32_t kCollapseOneBlock = 32768;
+
 void LbvhBuilder::collapse(hipStream_t s, uint32_t n, const Node* nodes, Node4* wide, uint32_t* numWide)
 {
     // the sort's second key buffer is free after the build: it holds the
     // breadth-first order of the wide nodes (at most n - 1 entries)
     const int numInternal = (int)std::max<uint32_t>(n, 2) - 1;
     k_wide_candidates<<<blocks_for(numInternal, 256), 256, 0, s>>>(nodes, numInternal, wideTmp);
+    if(n > kCollapseOneBlock) {
+        // free by now: both sort buffers, counters, leafParent and the boxes;
+        // nodeRange is this tree's (the build and the refit set it)
+        uint32_t* front = leafParent; // at most n / kSubtree nodes of more than kSubtree leaves at once
+        uint2* subtrees = reinterpret_cast<uint2*>(boxLo);
+        uint32_t* numSubtrees = sceneBox + 8;
+        k_level_init<<<blocks_for(numInternal, 256), 256, 0, s>>>(keysA, valsA, numInternal);
+        k_wide_levels_top<<<1, kDepthTopThreads, 0, s>>>(wideTmp, nodeRange, numInternal, keysA, front, front + n / 2, subtrees,
+                                                         numSubtrees);
+        k_wide_levels_sub<<<kDepthSubBlocks, kDepthSubThreads, 0, s>>>(wideTmp, numInternal, keysA, subtrees, numSubtrees);
+        sort_pass(s, keysA, valsA, keysB, valsB, (uint32_t)numInternal, 0, hist, counters);
+        k_wide_numbers<<<blocks_for(numInternal, 256), 256, 0, s>>>(valsB, hist, blocks_for(numInternal, kSortTile), numInternal,
+                                                                   counters, numWide);
+        k_wide_nodes<<<blocks_for(8u * (uint32_t)numInternal, 256), 256, 0, s>>>(wideTmp, valsB, counters, numWide, numInternal,
+                                                                                wide);
+        return;
+    }
     k_collapse_numbered<<<1, kCollapseThreads, 0, s>>>(wideTmp, numInternal, wide, reinterpret_cast<int32_t*>(keysB), numWide);
     k_wide_boxes<<<blocks_for(8u * (uint32_t)numInternal, 256), 256, 0, s>>>(wideTmp, reinterpret_cast<const int32_t*>(keysB),
                                                                              numWide, numInternal, wide);
