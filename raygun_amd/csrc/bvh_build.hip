@@ -444,6 +444,14 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t n, uint32_t v)
     if(i < n) p[i] = v;
 }
 
+// Two arrays, m <= n.
+__global__ void k_fill2_u32(uint32_t* p, uint32_t n, uint32_t* q, uint32_t m, uint32_t v)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if(i < n) p[i] = v;
+    if(i < m) q[i] = v;
+}
+
 // ---------------------------------------------------------------------------
 // 6. bottom-up refit
 // ---------------------------------------------------------------------------
@@ -453,12 +461,19 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t n, uint32_t v)
 // itself. The leaves are therefore cut into chunks of kRefitChunk
 // consecutive leaves: a workgroup finishes every node whose leaf range lies
 // inside its chunk with LDS counters and LDS copies of the child boxes, and
-// records each arrival at a node reaching outside the chunk. One workgroup
-// then finishes those upper nodes from the recorded arrivals (workgroup-scope
-// ordering only). A node's box is always fminf/fmaxf(slot 0, slot 1), so the
+// records each arrival at a node reaching outside the chunk. The same way a
+// workgroup per kRefitSuper leaves takes the arrivals recorded there as far as
+// nodes reaching outside those, and one workgroup finishes the rest
+// (workgroup-scope ordering only). A node's box is always fminf/fmaxf(slot 0, slot 1), so the
 // result does not depend on the order of arrival.
 constexpr int kRefitChunk = 1024;
 constexpr int kRefitTopThreads = 1024;
+// Without the middle pass one workgroup takes every arrival above the chunks:
+// 210 us for 1M triangles, where a rebuild with contact rays takes 1060 against
+// 910 us alone and 620 against 568 back to back. For 64k triangles the launch
+// costs more than it saves (145 against 149 us), for 200k as much.
+constexpr int kRefitSuper = 32 * kRefitChunk;
+constexpr uint32_t kRefitSuperMin = 1u << 18; // leaves from which on there is one
 
 __device__ __forceinline__ void write_slot(Node* nd, int slot, const float lo[3], const float hi[3])
 {
@@ -470,12 +485,13 @@ __device__ __forceinline__ void write_slot(Node* nd, int slot, const float lo[3]
     }
 }
 
-// counters[n - 1] counts the recorded arrivals, exits[] holds their nodes.
+// superCount[i] counts the arrivals recorded in leaves [i, i + 1) * superLeaves,
+// exits[i * superLeaves ..] holds their nodes (at most one per leaf).
 __global__ __launch_bounds__(kRefitChunk) void k_refit_chunk(const float4* __restrict__ boxLo, const float4* __restrict__ boxHi,
                                                              const uint32_t* __restrict__ leafPrim,
                                                              const uint32_t* __restrict__ leafParent,
-                                                             const uint2* __restrict__ range, Node* nodes, uint32_t* counters,
-                                                             uint32_t* exits, int n, float4* rootBox)
+                                                             const uint2* __restrict__ range, Node* nodes, uint32_t* superCount,
+                                                             uint32_t* exits, int n, float4* rootBox, uint32_t superLeaves)
 {
     __shared__ uint32_t cnt[kRefitChunk];
     __shared__ float box[kRefitChunk][12]; // node - c0: slot 0 lo, slot 1 lo, slot 0 hi, slot 1 hi
@@ -501,8 +517,9 @@ __global__ __launch_bounds__(kRefitChunk) void k_refit_chunk(const float4* __res
         write_slot(nd, slot, lo, hi);
         const int q = (int)p - c0; // a node lies inside its own leaf range
         if((int)r.x < c0 || (int)r.y > c1 || q < 0 || q >= kRefitChunk) {
-            // p reaches outside the chunk: the top pass takes it from here
-            const uint32_t e = atomicAdd(&counters[n - 1], 1u);
+            // p reaches outside the chunk: the next pass takes it from here
+            const uint32_t super = (uint32_t)c0 / superLeaves;
+            const uint32_t e = super * superLeaves + atomicAdd(&superCount[super], 1u);
             if(e < (uint32_t)n) exits[e] = p;
             return;
         }
@@ -527,15 +544,29 @@ __global__ __launch_bounds__(kRefitChunk) void k_refit_chunk(const float4* __res
     }
 }
 
-// The nodes above the chunks, from the recorded arrivals, in one workgroup.
-__global__ __launch_bounds__(kRefitTopThreads) void k_refit_top(Node* nodes, uint32_t* counters, const uint32_t* __restrict__ exits,
-                                                                int n, float4* rootBox)
+// The nodes above, from the arrivals recorded in a list (one workgroup each).
+// kTop: all of them; otherwise block i takes superchunk i's as far as nodes
+// within it and records the arrivals at others in topExits (topCount of them).
+template<bool kTop>
+__global__ __launch_bounds__(kRefitTopThreads) void k_refit_upper(Node* nodes, uint32_t* counters, const uint32_t* __restrict__ counts,
+                                                                  const uint32_t* exits, const uint2* __restrict__ range, int n,
+                                                                  float4* rootBox, uint32_t* topCount, uint32_t* topExits)
 {
-    const uint32_t numExits = min(counters[n - 1], (uint32_t)n);
+    const uint32_t first = kTop ? 0u : blockIdx.x * kRefitSuper;
+    const uint32_t last = kTop ? (uint32_t)n - 1u : min((uint32_t)n, first + kRefitSuper) - 1u; // last leaf
+    const uint32_t numExits = min(counts[blockIdx.x], last + 1u - first);
     for(uint32_t e = threadIdx.x; e < numExits; e += kRefitTopThreads) {
-        uint32_t p = exits[e];
+        uint32_t p = exits[first + e];
         for(int level = 0; level < 128; ++level) {
             if(p >= (uint32_t)(n - 1)) break;
+            if(!kTop) {
+                const uint2 r = range[p];
+                if(r.x < first || r.y > last) {
+                    const uint32_t at = atomicAdd(topCount, 1u);
+                    if(at < (uint32_t)n) topExits[at] = p;
+                    break;
+                }
+            }
             Node* nd = nodes + p;
             const uint32_t prev = __hip_atomic_fetch_add(&counters[p], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
             if(prev == 0u) break; // the other child's arrival finishes this node
@@ -1271,7 +1302,7 @@ __global__ void k_inst_gather(const float* __restrict__ w2o, const rgrt_instance
 // about twenty. The sort ranks each key by counting the keys that precede
 // it in (key, index) order, which is the order the stable radix sort
 // produces; the refit combines child boxes in the same order as
-// k_refit_chunk / k_refit_top (fminf/fmaxf of slot 0 and slot 1).
+// k_refit_chunk / k_refit_upper (fminf/fmaxf of slot 0 and slot 1).
 // The trees are therefore identical to the multi-kernel path's.
 // Instantiated for kMax = 256 and 1024 instances (one thread per instance):
 // the smaller form holds 28 KB of LDS instead of 116 KB, so with a frame's
@@ -1580,12 +1611,24 @@ void LbvhBuilder::build(hipStream_t s, uint32_t n, Node* nodes, uint32_t* leafPr
 
 void LbvhBuilder::refit_boxes(hipStream_t s, uint32_t n, const uint32_t* leafPrim, Node* nodes, float4* rootBox)
 {
-    // counters[0, n-1) per node, counters[n-1] the arrivals the top pass
-    // takes over; keysB (free after the sort) holds those arrivals
-    k_fill_u32<<<blocks_for(n, 256), 256, 0, s>>>(counters, n, 0u);
+    // counters[0, n - 1) per node; the arrivals' counts are in hist and their
+    // nodes in keysB and valsB, all free after the sort
+    const uint32_t superLeaves = n >= kRefitSuperMin ? (uint32_t)kRefitSuper : n;
+    const uint32_t supers = blocks_for(n, superLeaves);
+    uint32_t* superCount = hist;
+    uint32_t* topCount = hist + supers;
+    k_fill2_u32<<<blocks_for(n, 256), 256, 0, s>>>(counters, n, hist, supers + 1, 0u);
     k_refit_chunk<<<blocks_for(n, kRefitChunk), kRefitChunk, 0, s>>>(boxLo, boxHi, leafPrim, leafParent, nodeRange, nodes,
-                                                                     counters, keysB, (int)n, rootBox);
-    if(n > (uint32_t)kRefitChunk) k_refit_top<<<1, kRefitTopThreads, 0, s>>>(nodes, counters, keysB, (int)n, rootBox);
+                                                                     superCount, keysB, (int)n, rootBox, superLeaves);
+    if(n <= (uint32_t)kRefitChunk) return;
+    if(supers == 1) {
+        k_refit_upper<true><<<1, kRefitTopThreads, 0, s>>>(nodes, counters, superCount, keysB, nodeRange, (int)n, rootBox, nullptr,
+                                                           nullptr);
+        return;
+    }
+    k_refit_upper<false><<<supers, kRefitTopThreads, 0, s>>>(nodes, counters, superCount, keysB, nodeRange, (int)n, rootBox, topCount,
+                                                             valsB);
+    k_refit_upper<true><<<1, kRefitTopThreads, 0, s>>>(nodes, counters, topCount, valsB, nodeRange, (int)n, rootBox, nullptr, nullptr);
 }
 
 // Refit with the existing topology: new primitive boxes, same leaf order.
