@@ -16,7 +16,8 @@ uint32_t trace_resident_blocks();
 void launch_trace_queue_impl(hipStream_t s, const TraceScene& sc, const WavefrontState& st, int cur, uint32_t gridBlocks,
                              int32_t* spill, uint32_t* hostSlot, bool ahead);
 void launch_trace_rays_impl(hipStream_t s, const TraceScene& sc, const rgrt_ray* rays, uint32_t n, uint32_t cullMask,
-                            rgrt_hit* hits, const InstanceShade* inst, int32_t* spill, uint32_t gridBlocks);
+                            rgrt_hit* hits, const InstanceShade* inst, int32_t* spill, uint32_t gridBlocks, uint32_t simds,
+                            uint32_t* fetch);
 } // namespace rgrt
 
 using namespace rgrt;
@@ -201,6 +202,7 @@ struct rgrt_ctx {
     rgrt_ray* dRays = nullptr;
     rgrt_hit* dHits = nullptr;
     uint32_t rayCap = 0;
+    uint32_t* rayFetch = nullptr; // chunk counter of the ray queries
     size_t slotCap = 0;       // wavefront slots the slot arrays hold
     size_t sampleCap = 0;     // per-sample records the sample buffers hold
     uint32_t sampleGroups = 0; // most sample groups side by side (0: as many as fit)
@@ -975,6 +977,7 @@ rgrt_status rgrt_create(rgrt_ctx** out, const rgrt_config* cfg)
         check(hipGetDeviceProperties(&prop, c->device));
         c->numCUs = (uint32_t)std::max(1, prop.multiProcessorCount);
         c->apply_tuning();
+        dev_alloc(c->rayFetch, 1);
         for(int k = 0; k < 2; ++k) check(hipEventCreateWithFlags(&c->stageDone[k], hipEventDisableTiming));
         check(hipEventCreateWithFlags(&c->sceneEv, hipEventDisableTiming));
         if(cfg->width && cfg->height) alloc_images(c, cfg->width, cfg->height);
@@ -1024,6 +1027,7 @@ void rgrt_destroy(rgrt_ctx* c)
     dev_free(c->tlasRoot);
     dev_free(c->spill);
     dev_free(c->dRays);
+    dev_free(c->rayFetch);
     dev_free(c->dRgba8);
     dev_free(c->dHits);
     c->builder.release();
@@ -1402,7 +1406,7 @@ rgrt_status rgrt_trace_rays_device(rgrt_ctx* c, const rgrt_ray* rays, uint32_t n
     return guarded(c, [&]() {
         if(!c->haveTlas) return fail(c, RGRT_ERR_NOT_READY, "trace_rays: no TLAS");
         if(n && (!rays || !hits)) return fail(c, RGRT_ERR_INVALID_ARG, "trace_rays: null");
-        launch_trace_rays_impl(c->stream, c->scene(), rays, n, cullMask, hits, c->dShade, c->spill, c->traceGrid);
+        launch_trace_rays_impl(c->stream, c->scene(), rays, n, cullMask, hits, c->dShade, c->spill, c->traceGrid, 4 * c->numCUs, c->rayFetch);
         return RGRT_OK;
     });
 }
@@ -1419,7 +1423,8 @@ rgrt_status rgrt_trace_rays(rgrt_ctx* c, const rgrt_ray* rays, uint32_t n, uint3
         }
         if(!n) return RGRT_OK;
         check(hipMemcpyAsync(c->dRays, rays, n * sizeof(rgrt_ray), hipMemcpyHostToDevice, c->stream));
-        launch_trace_rays_impl(c->stream, c->scene(), c->dRays, n, cullMask, c->dHits, c->dShade, c->spill, c->traceGrid);
+        launch_trace_rays_impl(c->stream, c->scene(), c->dRays, n, cullMask, c->dHits, c->dShade, c->spill, c->traceGrid,
+                               4 * c->numCUs, c->rayFetch);
         check(hipMemcpyAsync(hits, c->dHits, n * sizeof(rgrt_hit), hipMemcpyDeviceToHost, c->stream));
         check(hipStreamSynchronize(c->stream));
         return traversal_errors(c);
