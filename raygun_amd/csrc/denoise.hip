@@ -7,14 +7,14 @@
 //
 // Layout: activations NHWC in bf16 with the channel count padded to a
 // multiple of 16; weights kept in fp32 (master copy, Adam moments) and
-// copied to bf16 in the two orders the convolutions read: [tap][cout][cin]
-// for the forward pass and [8 - tap][cin][cout] for the data gradient, which
-// makes the data gradient the same kernel as the forward convolution.
+// copied to bf16 twice in the order the convolution reads: for the forward
+// pass, and with mirrored taps and exchanged channels for the data gradient,
+// which makes the data gradient the same kernel as the forward convolution.
 //
 // Every convolution is an implicit GEMM on v_mfma_f32_16x16x32_bf16: a wave
-// computes 16 consecutive pixels of one row against all output channels,
-// K = 9 taps x input channels, one 16-byte load of 8 channels per lane and
-// operand. The weight gradient is the GEMM over pixels (K = pixels) per
+// computes strips of 16 consecutive pixels of one row against all output
+// channels, K = 9 taps x input channels, 8 channels per lane and operand, the
+// pixels read from a tile in LDS. The weight gradient is the GEMM over pixels (K = pixels) per
 // (tap, 16 input, 16 output channel) tile, summed over pixel chunks in a
 // fixed order, so training steps are deterministic.
 #include "rgrt_internal.h"
@@ -32,10 +32,10 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __host__ __device__ __forceinline__ uint16_t f2bf(float f)
 {
-    uint32_t u = __builtin_bit_cast(uint32_t, f);
-    if((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u); // NaN stays NaN
-    u += 0x7fffu + ((u >> 16) & 1u);                                           // round to nearest even
-    return (uint16_t)(u >> 16);
+    const uint32_t u = __builtin_bit_cast(uint32_t, f);
+    const uint32_t even = u + 0x7fffu + ((u >> 16) & 1u);                            // round to nearest even
+    const uint32_t r = (u & 0x7fffffffu) > 0x7f800000u ? u | 0x400000u : even; // NaN stays NaN
+    return (uint16_t)(r >> 16);
 }
 __host__ __device__ __forceinline__ float bf2f(uint16_t b) { return __builtin_bit_cast(float, (uint32_t)b << 16); }
 __device__ __forceinline__ float h2f(uint16_t b) { return (float)__builtin_bit_cast(_Float16, b); }
@@ -44,93 +44,194 @@ __device__ __forceinline__ uint16_t f2h(float x) { return __builtin_bit_cast(uin
 constexpr int kThreads = 256;
 constexpr int kConvStrips = 4; // 16-pixel strips a convolution wave computes (64 pixels of one row)
 
+// bf16 weights of a convolution of KIN to NOUT channels, whole K-steps of 32
+__host__ __device__ constexpr int conv_weights(int kin, int nout) { return (9 * kin + 31) / 32 * 32 * nout; }
+
 inline uint32_t grid_for(uint64_t n, uint32_t t) { return (uint32_t)((n + t - 1) / t); }
 
 // ---------------------------------------------------------------------------
-// Convolution 3x3, stride 1, zero padding 1: out = act(conv(in, wt) + bias)
-// in [N][H][W][KIN], wt [9][NOUT][KIN], out [N][H][W][NOUT]
+// Convolution 3x3, stride 1, zero padding 1: out = act(conv(in, w) + bias)
+// in [N][H][W][KIN], out [N][H][W][NOUT], w in the operand order of
+// k_prep_weights.
 // With C0 > 0 the input is the concatenation the decoder convolves (skip
 // connection): channels [0, C0) are the nearest 2x upsampling of
 // low [N][H/2][W/2][C0], channels [C0, KIN) come from in [N][H][W][KIN - C0];
 // the concatenated tensor is never stored.
+//
+// A workgroup computes 64 x 4R pixels (R rows a wave). It copies the pixels it
+// reads, border included, to LDS once, as planes of 8 channels, [plane][row]
+// [pixel] of 16 bytes each: the copy reads whole lines, writes the zeros of the
+// padding, so that the products need no bounds checks, and the 16 lanes that
+// read one operand's pixels read 256 consecutive bytes. Reading the operands
+// from memory for each tap instead was bound by the vector cache, which serves
+// a load of 64 lanes with strides of 32 to 128 bytes in about 50 cycles (a
+// consecutive one: 16), nine times per pixel.
+// The weights are the first operand: a lane then holds four consecutive
+// channels of one pixel, so that a strip of 16 pixels is stored whole.
+// Measured at 1920 x 1080, operands loaded from memory for each tap -> this
+// kernel: 16 to 16 channels 52 -> 33 us (133 MB, 4.0 TB/s), 48 to 16 156 -> 62,
+// 96 to 32 104 -> 42, 32 to 32 45 -> 22, 64 to 64 64 -> 24; the whole network
+// and its image kernels 786 -> 430 us. Four waves a SIMD hide a tile's copy
+// behind the products of the others; with two (all steps' operands loaded
+// ahead) the same code took as long as the loads from memory had.
 // ---------------------------------------------------------------------------
 template <int KIN, int NOUT, int C0 = 0>
-__global__ __launch_bounds__(kThreads) void k_conv(const uint16_t* __restrict__ in, const uint16_t* __restrict__ wt,
-                                                   const float* __restrict__ bias, uint16_t* __restrict__ out, int N, int H,
-                                                   int W, int relu, const uint16_t* __restrict__ low)
+struct ConvTile {
+    static constexpr int kRows = (NOUT == 16 && KIN <= 48) ? 2 : 1; // rows a wave: two where a row alone has few products
+    static constexpr int kH = kRows * (kThreads / 64), kW = 16 * kConvStrips;
+    static constexpr int kInPx = (kH + 2) * (kW + 2), kLowPx = (kH / 2 + 2) * (kW / 2 + 2);
+    static constexpr int kInChunks = (KIN - C0) / 8, kLowChunks = C0 / 8;
+    // bytes of a plane: the planes of one pixel are written together, to banks apart
+    static constexpr int plane(int px, int chunks) { return (px * 16 + 127) / 128 * 128 + (chunks ? 128 / chunks / 16 * 16 : 0); }
+    static constexpr int kInPlane = plane(kInPx, kInChunks), kLowPlane = plane(kLowPx, kLowChunks);
+    static constexpr int kLowAt = kInChunks * kInPlane;
+    static constexpr int kBytes = kLowAt + kLowChunks * kLowPlane;
+};
+
+// Pixels [y0, y0 + ROWS) x [x0, x0 + COLS) of an image of C channels to planes
+// of 8 channels in LDS; pixels outside of the image as zeros.
+template <int ROWS, int COLS, int C, int PLANE>
+__device__ __forceinline__ void conv_stage(const uint16_t* __restrict__ image, int y0, int x0, int H, int W, uint8_t* lds)
+{
+    constexpr int kChunks = C / 8, kCount = ROWS * COLS * kChunks, kTurns = (kCount + kThreads - 1) / kThreads;
+    u32x4 v[kTurns];
+    // every lane loads, from the image's border where its own pixel is outside
+    // of it: a load under a condition keeps the array out of registers
+#pragma unroll
+    for(int i = 0; i < kTurns; ++i) {
+        const int e = min((int)threadIdx.x + i * kThreads, kCount - 1);
+        const int px = e / kChunks, c = e % kChunks;
+        const int y = min(max(y0 + px / COLS, 0), H - 1), x = min(max(x0 + px % COLS, 0), W - 1);
+        v[i] = ld_global16(image + ((long)y * W + x) * C + 8 * c);
+    }
+#pragma unroll
+    for(int i = 0; i < kTurns; ++i) {
+        const int e = threadIdx.x + i * kThreads;
+        const int px = e / kChunks, c = e % kChunks;
+        const int y = y0 + px / COLS, x = x0 + px % COLS;
+        const bool isIn = y >= 0 && y < H && x >= 0 && x < W;
+        u32x4 t = v[i];
+#pragma unroll
+        for(int k = 0; k < 4; ++k) t[k] = isIn ? t[k] : 0u;
+        if(e < kCount) *reinterpret_cast<u32x4*>(lds + c * PLANE + px * 16) = t;
+    }
+}
+
+template <int KIN, int NOUT, int C0 = 0>
+__global__ __launch_bounds__(kThreads, NOUT > 64 ? 2 : 4) void k_conv(const uint16_t* __restrict__ in, const uint16_t* __restrict__ wt,
+                                                   const float* __restrict__ bias, uint16_t* __restrict__ out, int H, int W,
+                                                   int tilesX, int tilesY, int relu, const uint16_t* __restrict__ low)
 {
     static_assert(KIN % 16 == 0 && NOUT % 16 == 0, "channel counts are multiples of 16");
-    static_assert(C0 % 8 == 0 && C0 < KIN, "a load of 8 channels comes from one source");
+    static_assert(C0 % 8 == 0 && C0 < KIN, "an operand of 8 channels comes from one source");
+    using T = ConvTile<KIN, NOUT, C0>;
     constexpr int C1 = KIN - C0;
     constexpr int KT = 9 * KIN;
     constexpr int KSTEPS = (KT + 31) / 32;
     constexpr int NT = NOUT / 16;
-    constexpr int SPW = kConvStrips; // 16-pixel strips of one row per wave, sharing the weight operands
-    const int lane = threadIdx.x & 63;
-    const long wave = (long)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
-    const int stripsPerRow = (W + 15) / 16;
-    const int groupsPerRow = (stripsPerRow + SPW - 1) / SPW;
-    if(wave >= (long)N * H * groupsPerRow) return; // whole waves only
-    const int sg = (int)(wave % groupsPerRow);
-    const long row = wave / groupsPerRow;
-    const int y = (int)(row % H);
-    const int n = (int)(row / H);
+    constexpr int SPW = kConvStrips, R = T::kRows;
+    __shared__ __align__(16) uint8_t tile[T::kBytes];
+    const int tx = (int)(blockIdx.x % (unsigned)tilesX);
+    const int ty = (int)(blockIdx.x / (unsigned)tilesX % (unsigned)tilesY);
+    const int n = (int)(blockIdx.x / (unsigned)tilesX / (unsigned)tilesY);
+    const int x0 = tx * T::kW, y0 = ty * T::kH;
+    conv_stage<T::kH + 2, T::kW + 2, C1, T::kInPlane>(in + (long)n * H * W * C1, y0 - 1, x0 - 1, H, W, tile);
+    if constexpr(C0 > 0)
+        conv_stage<T::kH / 2 + 2, T::kW / 2 + 2, C0, T::kLowPlane>(low + (long)n * (H / 2) * (W / 2) * C0, y0 / 2 - 1,
+                                                                  x0 / 2 - 1, H / 2, W / 2, tile + T::kLowAt);
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int m = lane & 15, g = lane >> 4;
-    const int x0 = sg * SPW * 16 + m; // pixel of this lane in the group's first strip
-    f32x4 acc[SPW][NT];
+    if(y0 + wave * R >= H) return;
+    f32x4 acc[R][SPW][NT];
 #pragma unroll
-    for(int q = 0; q < SPW; ++q)
+    for(int r = 0; r < R; ++r)
 #pragma unroll
-        for(int j = 0; j < NT; ++j) acc[q][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for(int q = 0; q < SPW; ++q)
+#pragma unroll
+            for(int j = 0; j < NT; ++j) acc[r][q][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     const bf16x8 zero8 = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+    const uint16_t* wl = wt + lane * 8;
+    constexpr int kAheadSteps = 2; // K-steps whose weights are on the way
+    bf16x8 ahead[kAheadSteps][NT];
+#pragma unroll
+    for(int s = 0; s < kAheadSteps; ++s)
+#pragma unroll
+        for(int j = 0; j < NT; ++j) ahead[s][j] = __builtin_bit_cast(bf16x8, ld_global16(wl + (s * NT + j) * 512));
+    // lane group g reads the g-th 8 channels of a K-step
+    const int inLane = (wave * R * (T::kW + 2) + m) * 16 + g * T::kInPlane;
+    const int lowLane = T::kLowAt + g * T::kLowPlane;
+#pragma unroll
     for(int s = 0; s < KSTEPS; ++s) {
-        const int k0 = 32 * s + 8 * g;
-        const int tap = k0 / KIN;
-        const int c0 = k0 - tap * KIN;
-        const bool kin = k0 < KT;
-        const int yy = y + tap / 3 - 1;
-        const bool rowIn = kin && yy >= 0 && yy < H;
-        bf16x8 b[NT];
+        // all compile-time but for the lane group: from group `turn` on the
+        // channels are those of the next tap
+        constexpr int kChunks = KIN / 8;
+        const int tapA = 4 * s / kChunks, tapB = (4 * s + 3) / kChunks;
+        const int cA = 4 * s - tapA * kChunks, cB = 4 * s - tapB * kChunks; // + g: the 8 channels
+        const int turn = tapA == tapB ? 4 : -cB;
+        const bool later = g >= turn;
+        bf16x8 w[NT];
 #pragma unroll
         for(int j = 0; j < NT; ++j) {
-            b[j] = zero8;
-            if(kin) b[j] = __builtin_bit_cast(bf16x8, ld_global16(wt + ((long)tap * NOUT + 16 * j + m) * KIN + c0));
+            w[j] = ahead[s % kAheadSteps][j];
+            if(s + kAheadSteps < KSTEPS)
+                ahead[s % kAheadSteps][j] = __builtin_bit_cast(bf16x8, ld_global16(wl + ((s + kAheadSteps) * NT + j) * 512));
         }
-        bf16x8 a[SPW];
+#pragma unroll
+        for(int r = 0; r < R; ++r) {
+            const int offA = ((tapA / 3 + r) * (T::kW + 2) + tapA % 3) * 16 + (cA - C0 / 8) * T::kInPlane;
+            const int offB = ((tapB / 3 + r) * (T::kW + 2) + tapB % 3) * 16 + (cB - C0 / 8) * T::kInPlane;
+            int at = inLane + (later ? offB : offA), strip = 256;
+            if constexpr(C0 > 0) {
+                // rows and columns of the upsampled pixels, from the border's on
+                const int rowA = R == 2 ? wave + ((r + tapA / 3 - 1) >> 1) : (wave + tapA / 3 - 1) >> 1;
+                const int rowB = R == 2 ? wave + ((r + tapB / 3 - 1) >> 1) : (wave + tapB / 3 - 1) >> 1;
+                const int lowA = ((rowA + 1) * (T::kW / 2 + 2) + ((m + tapA % 3 - 1) >> 1) + 1) * 16 + cA * T::kLowPlane;
+                const int lowB = ((rowB + 1) * (T::kW / 2 + 2) + ((m + tapB % 3 - 1) >> 1) + 1) * 16 + cB * T::kLowPlane;
+                const bool fromLow = later ? cB + g < C0 / 8 : cA + g < C0 / 8;
+                at = fromLow ? lowLane + (later ? lowB : lowA) : at;
+                strip = fromLow ? 128 : 256;
+            }
+            const bool beyond = 4 * s + 3 >= 9 * kChunks && 4 * s + g >= 9 * kChunks; // past the last tap
+            if(beyond) at = 0; // any place of the tile
+#pragma unroll
+            for(int q = 0; q < SPW; ++q) {
+                bf16x8 a = *reinterpret_cast<const bf16x8*>(tile + at + q * strip);
+                if(beyond) a = zero8;
+#pragma unroll
+                for(int j = 0; j < NT; ++j) acc[r][q][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j], a, acc[r][q][j], 0, 0, 0);
+            }
+        }
+        // without it all steps' operands are loaded first, and spilled
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    float bv[NT][4];
+#pragma unroll
+    for(int j = 0; j < NT; ++j)
+#pragma unroll
+        for(int i = 0; i < 4; ++i) bv[j][i] = bias ? bias[16 * j + 4 * g + i] : 0.0f;
+    // lane holds D[row 4g + i][column m] of each strip: channel 16j + 4g + i of pixel m
+#pragma unroll
+    for(int r = 0; r < R; ++r) {
+        const int y = y0 + wave * R + r;
+        if(y >= H) break;
+        uint16_t* o = out + (((long)n * H + y) * W + x0 + m) * NOUT + 4 * g;
 #pragma unroll
         for(int q = 0; q < SPW; ++q) {
-            a[q] = zero8;
-            const int xx = x0 + 16 * q + tap % 3 - 1;
-            if(rowIn && xx >= 0 && xx < W) {
-                if(C0 > 0 && c0 < C0)
-                    a[q] = __builtin_bit_cast(bf16x8,
-                                              ld_global16(low + (((long)n * (H / 2) + yy / 2) * (W / 2) + xx / 2) * C0 + c0));
-                else
-                    a[q] = __builtin_bit_cast(bf16x8, ld_global16(in + (((long)n * H + yy) * W + xx) * C1 + (c0 - C0)));
+            if(x0 + 16 * q + m >= W) continue;
+#pragma unroll
+            for(int j = 0; j < NT; ++j) {
+                uint32_t b[4];
+#pragma unroll
+                for(int i = 0; i < 4; ++i) {
+                    float v = acc[r][q][j][i] + bv[j][i];
+                    if(relu) v = fmaxf(v, 0.0f);
+                    b[i] = f2bf(v);
+                }
+                *reinterpret_cast<u32x2*>(o + 16 * q * NOUT + 16 * j) = u32x2{b[0] | b[1] << 16, b[2] | b[3] << 16};
             }
         }
-#pragma unroll
-        for(int q = 0; q < SPW; ++q)
-#pragma unroll
-            for(int j = 0; j < NT; ++j) acc[q][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[q], b[j], acc[q][j], 0, 0, 0);
-    }
-    // lane holds D[row 4g + i][column m] of each strip: pixel 4g + i of the
-    // strip, channel 16j + m
-#pragma unroll
-    for(int j = 0; j < NT; ++j) {
-        const int co = 16 * j + m;
-        const float bv = bias ? bias[co] : 0.0f;
-#pragma unroll
-        for(int q = 0; q < SPW; ++q)
-#pragma unroll
-            for(int i = 0; i < 4; ++i) {
-                const int px = (sg * SPW + q) * 16 + 4 * g + i;
-                if(px < W) {
-                    float v = acc[q][j][i] + bv;
-                    if(relu) v = fmaxf(v, 0.0f);
-                    out[(((long)n * H + y) * W + px) * NOUT + co] = f2bf(v);
-                }
-            }
     }
 }
 
@@ -363,19 +464,26 @@ __global__ void k_adam(float* __restrict__ w, float* __restrict__ m, float* __re
     w[e] = w[e] - stepSize * mv / (sqrtf(vv) + eps);
 }
 
-// bf16 weight copies of one layer from the fp32 master [9][cin][cout]:
-// forward [tap][cout][cin], data gradient [8 - tap][cin][cout].
+// bf16 weight copies of one layer from the fp32 master [9][cin][cout], in the
+// order in which k_conv's lanes hold them: [K-step][16 outputs][lane][8], K =
+// (tap, input channel) padded with zeros to whole steps of 32. `wf`: the
+// layer itself; `wb`: its data gradient, taps mirrored, channels exchanged.
 __global__ void k_prep_weights(const float* __restrict__ w, int cin, int cout, uint16_t* __restrict__ wf,
                                uint16_t* __restrict__ wb)
 {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if(e >= 9 * cin * cout) return;
-    const int tap = e / (cin * cout);
-    const int r = e - tap * cin * cout;
-    const int ci = r / cout, co = r - (r / cout) * cout;
-    const uint16_t b = f2bf(w[e]);
-    wf[((long)tap * cout + co) * cin + ci] = b;
-    wb[((long)(8 - tap) * cin + ci) * cout + co] = b;
+    const int nf = conv_weights(cin, cout), nb = conv_weights(cout, cin);
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if(t >= nf + nb) return;
+    const bool back = t >= nf;
+    const int e = back ? t - nf : t;
+    const int kin = back ? cout : cin, nt = (back ? cin : cout) / 16;
+    const int lane = (e >> 3) & 63, block = e >> 9;
+    const int k = 32 * (block / nt) + 8 * (lane >> 4) + (e & 7);
+    const int o = 16 * (block % nt) + (lane & 15);
+    const int tap = k / kin, c = k - (k / kin) * kin;
+    float v = 0.0f;
+    if(tap < 9) v = back ? w[((long)(8 - tap) * cin + o) * cout + c] : w[((long)tap * cin + c) * cout + o];
+    (back ? wb : wf)[e] = f2bf(v);
 }
 
 // Network input from a frame of the stochastic mode: noisy RGB (BASE),
@@ -472,8 +580,10 @@ template <int KIN, int NOUT, int C0 = 0>
 void conv_t(hipStream_t s, const uint16_t* in, const uint16_t* wt, const float* bias, uint16_t* out, int N, int H, int W,
             int relu, const uint16_t* low = nullptr)
 {
-    const long waves = (long)N * H * (((W + 15) / 16 + kConvStrips - 1) / kConvStrips);
-    k_conv<KIN, NOUT, C0><<<grid_for(waves, kThreads / 64), kThreads, 0, s>>>(in, wt, bias, out, N, H, W, relu, low);
+    using T = ConvTile<KIN, NOUT, C0>;
+    const int tilesX = (W + T::kW - 1) / T::kW, tilesY = (H + T::kH - 1) / T::kH;
+    k_conv<KIN, NOUT, C0><<<(uint32_t)N * tilesX * tilesY, kThreads, 0, s>>>(in, wt, bias, out, H, W, tilesX, tilesY, relu,
+                                                                              low);
 }
 
 void conv(hipStream_t s, int kin, int nout, const uint16_t* in, const uint16_t* wt, const float* bias, uint16_t* out, int N,
@@ -486,8 +596,6 @@ void conv(hipStream_t s, int kin, int nout, const uint16_t* in, const uint16_t* 
     RGRT_CONV(32, 32)
     RGRT_CONV(32, 64)
     RGRT_CONV(64, 64)
-    RGRT_CONV(96, 32)
-    RGRT_CONV(48, 16)
     RGRT_CONV(16, 48)
     RGRT_CONV(32, 96)
     RGRT_CONV(64, 32)
@@ -556,17 +664,19 @@ Denoiser::Denoiser(uint32_t seed)
         off += kLayers[l].cout;
     }
     numParams = off;
-    size_t bfOff = 0;
+    size_t fwdOff = 0, bwdOff = 0;
     for(int l = 0; l < kNumLayers; ++l) {
-        wbfOff[l] = bfOff;
-        bfOff += 9ull * kLayers[l].cin * kLayers[l].cout;
+        wFwdOff[l] = fwdOff;
+        wBwdOff[l] = bwdOff;
+        fwdOff += conv_weights(kLayers[l].cin, kLayers[l].cout);
+        bwdOff += conv_weights(kLayers[l].cout, kLayers[l].cin);
     }
     check(hipMalloc(&params, numParams * 4));
     check(hipMalloc(&grads, numParams * 4));
     check(hipMalloc(&adamM, numParams * 4));
     check(hipMalloc(&adamV, numParams * 4));
-    check(hipMalloc(&wFwd, bfOff * 2));
-    check(hipMalloc(&wBwd, bfOff * 2));
+    check(hipMalloc(&wFwd, fwdOff * 2));
+    check(hipMalloc(&wBwd, bwdOff * 2));
     check(hipMemset(adamM, 0, numParams * 4));
     check(hipMemset(adamV, 0, numParams * 4));
     check(hipDeviceSynchronize()); // the fills are done before any stream's work reads them
@@ -602,9 +712,9 @@ Denoiser::~Denoiser()
 void Denoiser::prep_weights(hipStream_t s)
 {
     for(int l = 0; l < kNumLayers; ++l) {
-        const int n = 9 * kLayers[l].cin * kLayers[l].cout;
+        const int n = conv_weights(kLayers[l].cin, kLayers[l].cout) + conv_weights(kLayers[l].cout, kLayers[l].cin);
         k_prep_weights<<<grid_for(n, kThreads), kThreads, 0, s>>>(params + wOff[l], kLayers[l].cin, kLayers[l].cout,
-                                                                  wFwd + wbfOff[l], wBwd + wbfOff[l]);
+                                                                  wFwd + wFwdOff[l], wBwd + wBwdOff[l]);
     }
     weightsReady = true;
 }
@@ -670,7 +780,7 @@ void Denoiser::forward(hipStream_t s, int N, int H, int W, bool keepConcat)
 {
     if(!weightsReady) prep_weights(s);
     const int H1 = H / 2, W1 = W / 2, H2 = H / 4, W2 = W / 4;
-    auto w = [&](int l) { return wFwd + wbfOff[l]; };
+    auto w = [&](int l) { return wFwd + wFwdOff[l]; };
     auto b = [&](int l) { return params + bOff[l]; };
     conv(s, 16, 16, buf[X0], w(0), b(0), buf[A1], N, H, W, 1);
     conv(s, 16, 16, buf[A1], w(1), b(1), buf[S1], N, H, W, 1);
@@ -700,7 +810,7 @@ void Denoiser::backward(hipStream_t s, const float* target, int N, int H, int W)
     const long P0 = (long)N * H * W;
     const int H1 = H / 2, W1 = W / 2, H2 = H / 4, W2 = W / 4;
     const long P1 = P0 / 4, P2 = P0 / 16;
-    auto wb = [&](int l) { return wBwd + wbfOff[l]; };
+    auto wb = [&](int l) { return wBwd + wBwdOff[l]; };
     auto gw = [&](int l) { return grads + wOff[l]; };
     auto gb = [&](int l) { return grads + bOff[l]; };
     const int lossBlocks = (int)grid_for(P0, kThreads);

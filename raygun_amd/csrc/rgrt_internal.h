@@ -369,7 +369,7 @@ class Denoiser {
     void adam_step(hipStream_t s, float lr);
 
     size_t numParams = 0;
-    size_t wOff[kNumLayers], bOff[kNumLayers], wbfOff[kNumLayers];
+    size_t wOff[kNumLayers], bOff[kNumLayers], wFwdOff[kNumLayers], wBwdOff[kNumLayers];
     float *params = nullptr, *grads = nullptr, *adamM = nullptr, *adamV = nullptr;
     uint16_t *wFwd = nullptr, *wBwd = nullptr;
     bool weightsReady = false;

@@ -57,3 +57,31 @@ def test_infer_refuses_bad_sizes():
     finally:
         den.close()
         ctx.close()
+
+
+@pytest.mark.parametrize("shape", [(1, 4, 4), (1, 4, 64), (2, 8, 68), (1, 12, 128), (2, 20, 132), (1, 36, 260)])
+def test_tiles_and_their_remainders(shape):
+    """A workgroup computes a tile of 64 x 8 or 64 x 4 pixels: images smaller
+    than one, exactly one, and with remainders of one to three pixels, in both
+    directions and at all three levels of the network; more than one image."""
+    print(f"[case] denoiser tiles {shape}", flush=True)
+    n, h, w = shape
+    rng = np.random.default_rng(5)
+    x = rng.normal(0, 0.5, (n, h, w, 16)).astype(np.float32)
+    x[..., 11:] = 0.0
+    bits = (U.bf16(x).view(np.uint32) >> 16).astype(np.uint16)
+    params = U.init_params(9)
+    ctx = rgrt.Context(16, 16, 0)
+    den = rgrt.Denoiser(ctx, seed=1)
+    try:
+        den.set_params(params)
+        o = (den.infer(bits).astype(np.uint32) << 16).view(np.float32)
+    finally:
+        den.close()
+        ctx.close()
+    ref = U.Net(params, rounding=True).forward(U.bf16(x))["out"]
+    # bf16 storage after each of 11 layers, sums in another order: a value near a
+    # rounding boundary lands on its other side (2^-8 of itself) and travels on
+    rel = np.linalg.norm(o[..., :3] - ref[..., :3]) / np.linalg.norm(ref[..., :3])
+    assert rel < 1e-2, rel
+    assert np.abs(o[..., :3] - ref[..., :3]).max() < 11 * 2.0 ** -8 * np.abs(ref[..., :3]).max()
