@@ -203,8 +203,8 @@ struct rgrt_ctx {
     rgrt_hit* dHits = nullptr;
     uint32_t rayCap = 0;
     uint32_t* rayFetch = nullptr; // chunk counter of the ray queries
-    char* hRayIo = nullptr;       // pinned rays, hits and error word of small host queries (kPinnedRays)
-    char* hRayIoDev = nullptr;    // its device address
+    char* hRayIo = nullptr;       // pinned rays, hits and error word of small host queries (kPinnedRays),
+    char* hRayIoDev = nullptr;    // and its device address, both from rgrt_create on
     size_t slotCap = 0;       // wavefront slots the slot arrays hold
     size_t sampleCap = 0;     // per-sample records the sample buffers hold
     uint32_t sampleGroups = 0; // most sample groups side by side (0: as many as fit)
@@ -367,6 +367,23 @@ rgrt_status traversal_errors(rgrt_ctx* c)
     uint32_t flags = 0;
     check(hipMemcpy(&flags, c->st.counters + kTraversalErrorWord, 4, hipMemcpyDeviceToHost));
     return traversal_status(c, flags);
+}
+
+// Host queries of up to kPinnedRays rays: copies between pageable and device
+// memory and the read of the error word cost each some 10 us, more than the
+// bytes. The rays are read from, and hits and error word written to, pinned
+// memory of the context instead, with one wait: one ray 57 -> 35 us, 1,024
+// 97 -> 71, 4,096 123 -> 95 (hits through a device buffer and one more copy: 86
+// and 115).
+constexpr uint32_t kPinnedRays = 4096;
+constexpr size_t kRayIoHits = kPinnedRays * sizeof(rgrt_ray), kRayIoError = kRayIoHits + kPinnedRays * sizeof(rgrt_hit);
+
+// With the context, so that there is none without it and a first query costs
+// what later ones do.
+void alloc_ray_io(rgrt_ctx* c)
+{
+    check(hipHostMalloc((void**)&c->hRayIo, kRayIoError + 64, hipHostMallocMapped));
+    check(hipHostGetDevicePointer((void**)&c->hRayIoDev, c->hRayIo, 0));
 }
 
 template<typename F>
@@ -985,6 +1002,7 @@ rgrt_status rgrt_create(rgrt_ctx** out, const rgrt_config* cfg)
         c->numCUs = (uint32_t)std::max(1, prop.multiProcessorCount);
         c->apply_tuning();
         dev_alloc(c->rayFetch, 1);
+        alloc_ray_io(c);
         for(int k = 0; k < 2; ++k) check(hipEventCreateWithFlags(&c->stageDone[k], hipEventDisableTiming));
         check(hipEventCreateWithFlags(&c->sceneEv, hipEventDisableTiming));
         if(cfg->width && cfg->height) alloc_images(c, cfg->width, cfg->height);
@@ -1423,32 +1441,17 @@ rgrt_status rgrt_trace_rays_device(rgrt_ctx* c, const rgrt_ray* rays, uint32_t n
 
 namespace {
 
-// Host queries of up to kPinnedRays rays: copies between pageable and device
-// memory and the read of the error word cost each some 10 us, more than the
-// bytes. The rays are read from, and hits and error word written to, pinned
-// memory of the context instead, with one wait: one ray 57 -> 35 us, 1,024
-// 97 -> 71, 4,096 123 -> 95 (hits through a device buffer and one more copy: 86
-// and 115).
-constexpr uint32_t kPinnedRays = 4096;
-
 rgrt_status trace_few_rays(rgrt_ctx* c, const rgrt_ray* rays, uint32_t n, uint32_t cullMask, rgrt_hit* hits)
 {
-    constexpr size_t hitsAt = kPinnedRays * sizeof(rgrt_ray), errorAt = hitsAt + kPinnedRays * sizeof(rgrt_hit);
-    if(!c->hRayIo) {
-        char* p = nullptr;
-        check(hipHostMalloc((void**)&p, errorAt + 64, hipHostMallocMapped));
-        c->hRayIo = p;
-        check(hipHostGetDevicePointer((void**)&c->hRayIoDev, c->hRayIo, 0));
-    }
     std::memcpy(c->hRayIo, rays, n * sizeof(rgrt_ray));
     launch_trace_rays_impl(c->stream, c->scene(), reinterpret_cast<const rgrt_ray*>(c->hRayIoDev), n, cullMask,
-                           reinterpret_cast<rgrt_hit*>(c->hRayIoDev + hitsAt), c->dShade, c->spill, c->traceGrid, 4 * c->numCUs,
+                           reinterpret_cast<rgrt_hit*>(c->hRayIoDev + kRayIoHits), c->dShade, c->spill, c->traceGrid, 4 * c->numCUs,
                            c->rayFetch);
-    check(hipMemcpyAsync(c->hRayIo + errorAt, c->st.counters + kTraversalErrorWord, 4, hipMemcpyDeviceToHost, c->stream));
+    check(hipMemcpyAsync(c->hRayIo + kRayIoError, c->st.counters + kTraversalErrorWord, 4, hipMemcpyDeviceToHost, c->stream));
     check(hipStreamSynchronize(c->stream));
-    std::memcpy(hits, c->hRayIo + hitsAt, n * sizeof(rgrt_hit));
+    std::memcpy(hits, c->hRayIo + kRayIoHits, n * sizeof(rgrt_hit));
     uint32_t flags = 0;
-    std::memcpy(&flags, c->hRayIo + errorAt, 4);
+    std::memcpy(&flags, c->hRayIo + kRayIoError, 4);
     return traversal_status(c, flags);
 }
 

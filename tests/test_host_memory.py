@@ -1,0 +1,89 @@
+"""What the library's host side does when memory runs out, on a HIP runtime in
+host memory (fake_hip.cpp: allocations can be made to fail, kernels do not
+run): a failed call returns an error and leaves nothing behind that a later
+call would hand to a kernel. CPU only."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PREAMBLE = """
+import ctypes, sys
+sys.path.insert(0, {root!r})
+F = ctypes.CDLL({fake!r}, ctypes.RTLD_GLOBAL)  # before librgrt.so: its symbols come first
+F.fake_log.restype = ctypes.c_char_p
+import numpy as np
+from raygun_amd import rgrt
+from raygun_amd.records import INSTANCE, RAY, VERTEX
+from raygun_amd.rgrt import Context, RgrtError
+
+def log():
+    return F.fake_log().decode().split("\\n")
+
+def launches(name):
+    return [l.split() for l in log() if l.startswith("launch") and name in l]
+
+def allocations(name="hipMalloc"):
+    return [int(l.split()[1]) for l in log() if l.startswith(name + " ")]
+
+def fail(name, nth=1):
+    F.fake_fail(name.encode(), nth)
+
+def raises(f):
+    try:
+        f()
+    except RgrtError as e:
+        return str(e)
+    raise AssertionError("no error")
+
+def one_triangle(ctx):
+    v = np.zeros(3, VERTEX)
+    v["position"] = [[0, 0, 0], [1, 0, 0], [0, 1, 0]]
+    ctx.upload_geometry(v, np.arange(3))
+    inst = np.zeros(1, INSTANCE)
+    inst["blas"] = ctx.build_blas(0, 0, 1, 3)
+    inst["transform"] = [1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 0]
+    inst["mask"] = 0xFF
+    ctx.build_tlas(inst)
+    return inst
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    fake = str(tmp_path_factory.mktemp("fake_hip") / "fake_hip.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(HERE, "fake_hip.cpp"), "-o", fake], check=True)
+
+    def go(body):
+        r = subprocess.run([sys.executable, "-c", PREAMBLE.format(root=ROOT, fake=fake) + body], capture_output=True, text=True,
+                           timeout=120)
+        assert r.returncode == 0, r.stdout + r.stderr
+
+    return go
+
+
+def test_pinned_ray_memory_without_a_device_address(run):
+    """The pinned buffer of small host queries is there with its device
+    address or not at all: no query runs on a null one."""
+    run("""
+fail("hipHostGetDevicePointer")
+try:
+    ctx = Context(16, 16)
+except RgrtError:
+    ctx = Context(16, 16)
+else:
+    one_triangle(ctx)
+    raises(lambda: ctx.trace_rays(np.zeros(1, RAY)))
+    log()
+    ctx.trace_rays(np.zeros(1, RAY))
+    assert allocations("hipHostMalloc"), "a query after the failed one ran without the buffer"
+one_triangle(ctx)
+log()
+ctx.trace_rays(np.zeros(4, RAY))
+assert len(launches("k_trace_rays")) == 1
+""")
