@@ -202,7 +202,7 @@ struct rgrt_ctx {
     rgrt_ray* dRays = nullptr;
     rgrt_hit* dHits = nullptr;
     uint32_t rayCap = 0;
-    uint32_t* rayFetch = nullptr; // chunk counter of the ray queries
+    uint32_t* rayFetch = nullptr; // chunk counter of the ray queries, error word of a context without images
     char* hRayIo = nullptr;       // pinned rays, hits and error word of small host queries (kPinnedRays),
     char* hRayIoDev = nullptr;    // and its device address, both from rgrt_create on
     size_t slotCap = 0;       // wavefront slots the slot arrays hold
@@ -239,9 +239,11 @@ struct rgrt_ctx {
         sc.numInstances = haveTlas ? numInstances : 0;
         sc.tlasNodeCap = std::max<uint32_t>(sc.numInstances, 2u) - 1u;
         sc.numBlas = (uint32_t)sd->blas.size();
-        sc.errors = st.counters + kTraversalErrorWord;
+        sc.errors = error_word();
         return sc;
     }
+    // Where the traversal kernels flag bad indices.
+    uint32_t* error_word() const { return st.counters ? st.counters + kTraversalErrorWord : rayFetch + 1; }
 };
 
 namespace {
@@ -365,7 +367,7 @@ rgrt_status traversal_status(rgrt_ctx* c, uint32_t flags)
 rgrt_status traversal_errors(rgrt_ctx* c)
 {
     uint32_t flags = 0;
-    check(hipMemcpy(&flags, c->st.counters + kTraversalErrorWord, 4, hipMemcpyDeviceToHost));
+    check(hipMemcpy(&flags, c->error_word(), 4, hipMemcpyDeviceToHost));
     return traversal_status(c, flags);
 }
 
@@ -1001,7 +1003,8 @@ rgrt_status rgrt_create(rgrt_ctx** out, const rgrt_config* cfg)
         check(hipGetDeviceProperties(&prop, c->device));
         c->numCUs = (uint32_t)std::max(1, prop.multiProcessorCount);
         c->apply_tuning();
-        dev_alloc(c->rayFetch, 1);
+        dev_alloc(c->rayFetch, 2);
+        check(hipMemsetAsync(c->rayFetch, 0, 8, c->stream));
         alloc_ray_io(c);
         for(int k = 0; k < 2; ++k) check(hipEventCreateWithFlags(&c->stageDone[k], hipEventDisableTiming));
         check(hipEventCreateWithFlags(&c->sceneEv, hipEventDisableTiming));
@@ -1447,7 +1450,7 @@ rgrt_status trace_few_rays(rgrt_ctx* c, const rgrt_ray* rays, uint32_t n, uint32
     launch_trace_rays_impl(c->stream, c->scene(), reinterpret_cast<const rgrt_ray*>(c->hRayIoDev), n, cullMask,
                            reinterpret_cast<rgrt_hit*>(c->hRayIoDev + kRayIoHits), c->dShade, c->spill, c->traceGrid, 4 * c->numCUs,
                            c->rayFetch);
-    check(hipMemcpyAsync(c->hRayIo + kRayIoError, c->st.counters + kTraversalErrorWord, 4, hipMemcpyDeviceToHost, c->stream));
+    check(hipMemcpyAsync(c->hRayIo + kRayIoError, c->error_word(), 4, hipMemcpyDeviceToHost, c->stream));
     check(hipStreamSynchronize(c->stream));
     std::memcpy(hits, c->hRayIo + kRayIoHits, n * sizeof(rgrt_hit));
     uint32_t flags = 0;

@@ -87,3 +87,14 @@ log()
 ctx.trace_rays(np.zeros(4, RAY))
 assert len(launches("k_trace_rays")) == 1
 """)
+
+
+@pytest.mark.parametrize("rays", [1, 5000])
+def test_ray_queries_without_images(run, rays):
+    """A context of size 0 x 0 answers ray queries: the error word of the
+    traversal is there without a frame's counters."""
+    run(f"""
+ctx = Context(0, 0)
+one_triangle(ctx)
+assert len(ctx.trace_rays(np.zeros({rays}, RAY))) == {rays}
+""")
