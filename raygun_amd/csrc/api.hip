@@ -634,7 +634,7 @@ void prepare_sample_groups(rgrt_ctx* c)
         dev_alloc(s.rays[0], slots * kRayWords);
         dev_alloc(s.rays[1], slots * kRayWords);
         dev_alloc(s.hits, slots * kHitWords);
-        dev_alloc(s.ahead, ahead_words(slots));
+        if(ahead_words(slots) > ahead_words(c->slotCap)) dev_alloc(s.ahead, ahead_words(slots));
         c->slotCap = slots;
     }
     if(g > 1 && (size_t)n * s.nimg > c->sampleCap) {

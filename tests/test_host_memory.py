@@ -18,7 +18,7 @@ F = ctypes.CDLL({fake!r}, ctypes.RTLD_GLOBAL)  # before librgrt.so: its symbols 
 F.fake_log.restype = ctypes.c_char_p
 import numpy as np
 from raygun_amd import rgrt
-from raygun_amd.records import INSTANCE, RAY, VERTEX
+from raygun_amd.records import INSTANCE, RAY, UBO, VERTEX
 from raygun_amd.rgrt import Context, RgrtError
 
 def log():
@@ -97,4 +97,21 @@ def test_ray_queries_without_images(run, rays):
 ctx = Context(0, 0)
 one_triangle(ctx)
 assert len(ctx.trace_rays(np.zeros({rays}, RAY))) == {rays}
+""")
+
+
+def test_first_frame_of_several_samples_keeps_the_queue_of_rays_ahead(run):
+    """The slot arrays grow with the samples; the queue of rays ahead has one
+    size from 300,000 slots on and is not allocated again."""
+    run("""
+ctx = Context(800, 600)
+queue = 300000 * 2 * 7 * 4
+assert queue in allocations()
+inst = one_triangle(ctx)
+ubo = np.zeros((), UBO)
+ubo["numSamples"], ubo["maxRecursions"] = 3, 1
+log()
+ctx.frame(ubo, inst)
+grown = allocations()
+assert 3 * 800 * 600 * 10 * 4 in grown and queue not in grown, grown
 """)
