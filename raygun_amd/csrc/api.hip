@@ -42,6 +42,9 @@ void dev_free(T*& p)
     p = nullptr;
 }
 
+// Frees p and allocates it anew. A buffer's recorded capacity is set to zero
+// before it grows: if memory runs out, p is null, the call reports it, and the
+// next call allocates again instead of handing the null to a kernel.
 template<typename T>
 void dev_alloc(T*& p, size_t count)
 {
@@ -193,6 +196,7 @@ struct rgrt_ctx {
                 check(hipStreamSynchronize(stream));
                 check(hipFree(spill));
                 spill = nullptr;
+                spillBytes = 0;
             }
             check(hipMalloc((void**)&spill, need));
             spillBytes = need;
@@ -434,6 +438,8 @@ void free_images(rgrt_ctx* c)
     c->sampleCap = 0;
     dev_free(s.counters);
     s.npix = 0;
+    c->w = 0;
+    c->h = 0;
 }
 
 // Whether a frame's shading passes queue reflection and refraction rays ahead
@@ -487,7 +493,6 @@ void alloc_images(rgrt_ctx* c, uint32_t w, uint32_t h)
     s.nimg = (uint32_t)npix;
     s.groups = 1;
     s.numSamples = 1;
-    c->slotCap = npix;
     dev_alloc(s.payload, npix * kPayloadWords);
     dev_alloc(s.accum, npix * kAccumWords);
     dev_alloc(s.lum2, npix);
@@ -499,6 +504,7 @@ void alloc_images(rgrt_ctx* c, uint32_t w, uint32_t h)
     dev_alloc(s.segs, kMaxBands * kSegmentBlock);
     dev_alloc(s.counters, 64);
     check(hipMemsetAsync(s.counters, 0, 64 * 4, c->stream));
+    c->slotCap = npix;
     c->w = w;
     c->h = h;
 }
@@ -528,6 +534,8 @@ void ensure_inst_cap(rgrt_ctx* c, uint32_t n)
     if(n <= c->instCap) return;
     check(hipStreamSynchronize(c->stream)); // queued frames still use the old buffers
     const uint32_t cap = std::max<uint32_t>(n, 64);
+    c->instCap = 0;
+    c->haveTlas = false; // it is freed here
     for(int k = 0; k < 2; ++k) {
         if(c->hInstStage[k]) {
             check(hipEventSynchronize(c->stageDone[k]));
@@ -555,6 +563,8 @@ void ensure_host_counts(rgrt_ctx* c, uint32_t n)
     if(c->hostCounts) {
         check(hipStreamSynchronize(c->stream));
         (void)hipHostFree(c->hostCounts);
+        c->hostCounts = nullptr;
+        c->hostCountsCap = 0;
     }
     const uint32_t cap = std::max<uint32_t>(n, 1024);
     check(hipHostMalloc((void**)&c->hostCounts, cap * 4, hipHostMallocMapped));
@@ -629,16 +639,19 @@ void prepare_sample_groups(rgrt_ctx* c)
     const size_t slots = (size_t)s.nimg * g;
     if(slots > c->slotCap) {
         check(hipStreamSynchronize(c->stream)); // queued frames still use the old arrays
+        const size_t had = c->slotCap;
+        c->slotCap = 0;
         dev_alloc(s.payload, slots * kPayloadWords);
         dev_alloc(s.frames, frame_words(slots));
         dev_alloc(s.rays[0], slots * kRayWords);
         dev_alloc(s.rays[1], slots * kRayWords);
         dev_alloc(s.hits, slots * kHitWords);
-        if(ahead_words(slots) > ahead_words(c->slotCap)) dev_alloc(s.ahead, ahead_words(slots));
+        if(ahead_words(slots) > ahead_words(had)) dev_alloc(s.ahead, ahead_words(slots));
         c->slotCap = slots;
     }
     if(g > 1 && (size_t)n * s.nimg > c->sampleCap) {
         check(hipStreamSynchronize(c->stream));
+        c->sampleCap = 0;
         dev_alloc(s.sampleAcc, (size_t)n * s.nimg * kAccumWords);
         dev_alloc(s.sampleLum2, (size_t)n * s.nimg);
         c->sampleCap = (size_t)n * s.nimg;
@@ -1469,6 +1482,7 @@ rgrt_status rgrt_trace_rays(rgrt_ctx* c, const rgrt_ray* rays, uint32_t n, uint3
         if(n && (!rays || !hits)) return fail(c, RGRT_ERR_INVALID_ARG, "trace_rays: null");
         if(n && n <= kPinnedRays) return trace_few_rays(c, rays, n, cullMask, hits);
         if(n > c->rayCap) {
+            c->rayCap = 0;
             dev_alloc(c->dRays, n);
             dev_alloc(c->dHits, n);
             c->rayCap = n;
@@ -2303,7 +2317,7 @@ rgrt_status rgrt_read_image_rgba8(rgrt_ctx* c, rgrt_image which, rgrt_format for
         const uint64_t npix = (uint64_t)c->w * c->h;
         if(bytes != npix * 4 || !dst) return fail(c, RGRT_ERR_INVALID_ARG, "read_image_rgba8: size mismatch");
         if(c->rgba8Cap < npix) {
-            dev_free(c->dRgba8);
+            c->rgba8Cap = 0;
             dev_alloc(c->dRgba8, npix * 4);
             c->rgba8Cap = npix;
         }

@@ -768,6 +768,7 @@ void Denoiser::reserve(int N, int H, int W, bool training)
     if(bytes > wsBytes) {
         if(ws) check(hipFree(ws));
         ws = nullptr;
+        wsBytes = 0;
         check(hipMalloc(&ws, bytes));
         wsBytes = bytes;
     }

@@ -115,3 +115,58 @@ ctx.frame(ubo, inst)
 grown = allocations()
 assert 3 * 800 * 600 * 10 * 4 in grown and queue not in grown, grown
 """)
+
+
+GROWING = {
+    # (a call, the same on something larger, the allocation that fails)
+    "rays": ("ctx.trace_rays(np.zeros(5000, RAY))", "ctx.trace_rays(np.zeros(9000, RAY))", "hipMalloc", 2),
+    "slots": ("frame(1)", "frame(3)", "hipMalloc", 2),
+    "sample records": ("frame(2)", "frame(3)", "hipMalloc", 6),
+    "pass counts": ("ctx.set_sample_groups(1); frame(1)", "frame(3, 7)", "hipHostMalloc", 1),
+    "images": ("ctx.resize(16, 16); frame(1)", "ctx.resize(24, 24)", "hipMalloc", 3),
+    "8-bit image": ("ctx.resize(16, 16); ctx.read_image_rgba8()", "ctx.resize(24, 24); log(); fail('hipMalloc'); ctx.read_image_rgba8()",
+                    "", 0),
+    "instances": ("ctx.build_tlas(inst); ctx.trace_rays(np.zeros(1, RAY))", "ctx.build_tlas(np.repeat(inst, 100))", "hipMalloc", 3),
+    "stack spill": ("ctx.set_tuning(drainBlocksPerCU=4)", "ctx.set_tuning(drainBlocksPerCU=32)", "hipMalloc", 1),
+    "network": ("den.infer(np.zeros((1, 16, 16, 16)))", "den.infer(np.zeros((1, 64, 64, 16)))", "hipMalloc", 1),
+}
+
+
+@pytest.mark.parametrize("what", GROWING)
+def test_a_buffer_that_could_not_grow_is_allocated_by_the_next_call(run, what):
+    """What was freed to make room is not taken for what it was: the smaller
+    call allocates again and succeeds."""
+    small, large, function, nth = GROWING[what]
+    run(f"""
+ctx = Context(16, 16)
+inst = one_triangle(ctx)
+den = rgrt.Denoiser(ctx)
+den.set_params(den.get_params())
+
+def frame(samples, recursions=1):
+    ubo = np.zeros((), UBO)
+    ubo["numSamples"], ubo["maxRecursions"] = samples, recursions
+    ctx.frame(ubo, inst)
+
+def small():
+    {small}
+
+def large():
+    {large}
+
+small()
+if {function!r}:
+    fail({function!r}, {nth})
+assert "out of memory" in raises(large)
+if {what!r} == "instances":
+    assert "no TLAS" in raises(lambda: ctx.trace_rays(np.zeros(1, RAY)))
+if {what!r} == "images":
+    assert "zero-sized" in raises(lambda: frame(1))
+log()
+small()
+l = log()
+assert any(x.startswith("hipMalloc") or x.startswith("hipHostMalloc") for x in l), l
+log()
+small()
+assert not allocations()
+""")
