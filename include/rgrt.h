@@ -521,7 +521,8 @@ typedef struct rgrt_stats {
 typedef struct rgrt_tuning {
     uint32_t wavefrontPasses;   /* wavefront passes before the persistent drain takes the tail
                                    (0 = drain everything, >= 64 = never drain)                */
-    uint32_t traceBlocksPerCU;  /* persistent traversal grid, blocks of 256 per CU            */
+    uint32_t traceBlocksPerCU;  /* persistent traversal grid, blocks of 256 per CU; more than a
+                                   CU holds at once (5) are taken as that many                */
     uint32_t shadeBlocksPerCU;  /* shading grid, blocks of 256 per CU                         */
     uint32_t drainBlocksPerCU;  /* drain grid, blocks of 256 per CU                           */
     uint32_t hostLag;           /* wavefront passes the GPU may run ahead of the host's check
@@ -539,7 +540,8 @@ typedef struct rgrt_tuning {
 
 /* Sets / reads the launch shape (defaults tuned for MI355X). Values outside
  * 1..32 blocks per CU, a hostLag outside 1..16 or more than 4 frameBands
- * are rejected. */
+ * are rejected. What is read is the shape launched: a traceBlocksPerCU above
+ * what a CU holds reads back as what it holds. */
 rgrt_status rgrt_set_tuning(rgrt_ctx* ctx, const rgrt_tuning* t);
 rgrt_status rgrt_get_tuning(rgrt_ctx* ctx, rgrt_tuning* t);
 /* No counterpart in the reference (its raygen loops over a pixel's samples,

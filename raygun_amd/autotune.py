@@ -2,7 +2,9 @@
 drain, persistent grid sizes per CU, host lag) for one scene by timing its
 frames with hipEvents. Coordinate descent: each parameter in turn takes the
 value from its candidate list that gives the fastest frame with the others
-fixed, for `rounds` rounds. Every candidate is a documented launch shape, so
+fixed, for `rounds` rounds. A candidate the library launches as another shape
+(more blocks than a CU holds) counts as that one and is not timed twice. Every
+candidate is a documented launch shape, so
 a sweep only changes timing, never results (the tests render the same frame
 under different tunings and compare).
 
@@ -13,7 +15,7 @@ from .hiptime import HipEvents, time_ms
 
 CANDIDATES = {
     "wavefrontPasses": [2, 4, 6, 8, 12],
-    "traceBlocksPerCU": [4, 6, 8],
+    "traceBlocksPerCU": [3, 4, 5],
     "shadeBlocksPerCU": [4, 8, 12],
     "drainBlocksPerCU": [2, 4, 8],
     "hostLag": [1, 2, 4],
@@ -49,13 +51,15 @@ def tune(ctx, frame, candidates=None, rounds=1, reps=2, log=None, contexts=None,
     table = [(dict(best), best_ms)]
     for _ in range(rounds):
         for name, values in cand.items():
-            current = best[name]  # already timed with the other parameters as they are
+            timed = [best]  # shapes timed with the other parameters as they are
             for v in values:
-                if v == current:
-                    continue
                 t = dict(best)
                 t[name] = v
                 apply(t)
+                t = dict(ctx.tuning())
+                if t in timed:
+                    continue
+                timed.append(t)
                 ms = measure()
                 table.append((t, ms))
                 if log:

@@ -158,7 +158,7 @@ struct rgrt_ctx {
     int32_t* spill = nullptr;
     size_t spillBytes = 0;
     uint32_t traceGrid = 0, shadeGrid = 0, drainGrid = 0;
-    rgrt_tuning tuning{6, 6, 8, 4, 2, 1}; // measured on config 2 (1080p, 2M triangles)
+    rgrt_tuning tuning{6, 5, 8, 4, 2, 1}; // measured on config 2 (1080p, 2M triangles)
     rgrt_sampling sampling{RGRT_SAMPLING_WHITTED, 0u, {0u, 0u}};
     hipEvent_t evDrainStart = nullptr, evDrainEnd = nullptr;
     bool lastDrained = false;
@@ -184,7 +184,8 @@ struct rgrt_ctx {
         // the traversal grid is persistent: blocks past what a CU holds would
         // start on their share when the others are done (4K at 4 samples with
         // six blocks per CU, five of them resident: 95.8 ms, clamped 86.0)
-        traceGrid = numCUs * std::min(tuning.traceBlocksPerCU, trace_resident_blocks());
+        tuning.traceBlocksPerCU = std::min(tuning.traceBlocksPerCU, trace_resident_blocks());
+        traceGrid = numCUs * tuning.traceBlocksPerCU;
         shadeGrid = numCUs * tuning.shadeBlocksPerCU;
         drainGrid = numCUs * tuning.drainBlocksPerCU;
         bands = std::max<uint32_t>(1u, std::min(tuning.frameBands, kMaxBands));

@@ -66,6 +66,20 @@ def test_autotune_confirmation_discards_a_lucky_timing():
         assert sum(seen.values()) == 3 + (3 * 2 if confirm else 0)
 
 
+def test_autotune_times_a_shape_once():
+    """The library launches at most as many blocks per CU as a CU holds and
+    reads back what it launches: candidates above are one shape, timed once
+    and reported as what ran."""
+    class Holds5(_FakeContext):
+        def set_tuning(self, **t):
+            super().set_tuning(**{**t, "traceBlocksPerCU": min(t["traceBlocksPerCU"], 5)})
+
+    ctx = Holds5({"wavefrontPasses": 6, "traceBlocksPerCU": 4})
+    best, ms, table = autotune.tune(ctx, None, candidates={"traceBlocksPerCU": [4, 6, 7, 8]}, timer=lambda: 10.0 - ctx.t["traceBlocksPerCU"])
+    assert [t["traceBlocksPerCU"] for t, _ in table] == [4, 5]
+    assert best == ctx.t == {"wavefrontPasses": 6, "traceBlocksPerCU": 5} and ms == 5.0
+
+
 def test_batched_scene_sizes_are_seeded_and_clipped():
     a = batched.scene_sizes(32, 3)
     assert a == batched.scene_sizes(32, 3)

@@ -1,7 +1,7 @@
-"""What the library's host side does when memory runs out, on a HIP runtime in
-host memory (fake_hip.cpp: allocations can be made to fail, kernels do not
-run): a failed call returns an error and leaves nothing behind that a later
-call would hand to a kernel. CPU only."""
+"""The library's host side on a HIP runtime in host memory (fake_hip.cpp:
+allocations can be made to fail, kernels do not run): what it allocates and
+launches, and that a call that runs out of memory returns an error and leaves
+nothing behind that a later call would hand to a kernel. CPU only."""
 import os
 import subprocess
 import sys
@@ -169,4 +169,25 @@ assert any(x.startswith("hipMalloc") or x.startswith("hipHostMalloc") for x in l
 log()
 small()
 assert not allocations()
+""")
+
+
+@pytest.mark.parametrize("holds", [3, 5, 40])
+def test_launch_shape_reads_back_as_launched(run, holds):
+    """traceBlocksPerCU beyond what a CU holds is what it holds, in the grid
+    and in what rgrt_get_tuning says."""
+    run(f"""
+F.fake_occupancy({holds})
+ctx = Context(16, 16)
+inst = one_triangle(ctx)
+ubo = np.zeros((), UBO)
+ubo["numSamples"], ubo["maxRecursions"] = 1, 1
+assert ctx.tuning()["traceBlocksPerCU"] == min(5, {holds})
+for blocks in (1, 4, 8, 32):
+    ctx.set_tuning(traceBlocksPerCU=blocks)
+    assert ctx.tuning()["traceBlocksPerCU"] == min(blocks, {holds})
+    log()
+    ctx.frame(ubo, inst)
+    grids = [int(l[2]) for l in launches("k_trace_queue")]
+    assert grids and all(g == 2 * min(blocks, {holds}) for g in grids), grids  # two CUs
 """)
