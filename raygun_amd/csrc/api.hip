@@ -2191,11 +2191,6 @@ rgrt_status rgrt_denoiser_set_params(rgrt_denoiser* den, const float* params, ui
     });
 }
 
-// The backward pass (and so training) is switched off: its first GPU run
-// faulted in the weight-gradient kernel (an address beyond the legal range)
-// and no out-of-bounds access has been found in any of its kernels, so it
-// stays off the GPU until a cause is shown.
-constexpr bool kDenoiserBackwardEnabled = false;
 constexpr const char* kDenoiserBackwardOff =
     "the denoiser's backward pass is switched off: its weight-gradient kernel faulted the GPU and no cause has been "
     "found yet";

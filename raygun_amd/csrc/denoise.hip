@@ -7,9 +7,10 @@
 //
 // Layout: activations NHWC in bf16 with the channel count padded to a
 // multiple of 16; weights kept in fp32 (master copy, Adam moments) and
-// copied to bf16 twice in the order the convolution reads: for the forward
-// pass, and with mirrored taps and exchanged channels for the data gradient,
-// which makes the data gradient the same kernel as the forward convolution.
+// copied to bf16 in the order the convolution reads (conv_weights.h): for the
+// forward pass, and where training is enabled with mirrored taps and exchanged
+// channels for the data gradient, which makes the data gradient the same
+// kernel as the forward convolution.
 //
 // Every convolution is an implicit GEMM on v_mfma_f32_16x16x32_bf16: a wave
 // computes strips of 16 consecutive pixels of one row against all output
@@ -17,6 +18,7 @@
 // pixels read from a tile in LDS. The weight gradient is the GEMM over pixels (K = pixels) per
 // (tap, 16 input, 16 output channel) tile, summed over pixel chunks in a
 // fixed order, so training steps are deterministic.
+#include "conv_weights.h"
 #include "rgrt_internal.h"
 
 #include <cmath>
@@ -44,15 +46,11 @@ __device__ __forceinline__ uint16_t f2h(float x) { return __builtin_bit_cast(uin
 constexpr int kThreads = 256;
 constexpr int kConvStrips = 4; // 16-pixel strips a convolution wave computes (64 pixels of one row)
 
-// bf16 weights of a convolution of KIN to NOUT channels, whole K-steps of 32
-__host__ __device__ constexpr int conv_weights(int kin, int nout) { return (9 * kin + 31) / 32 * 32 * nout; }
-
 inline uint32_t grid_for(uint64_t n, uint32_t t) { return (uint32_t)((n + t - 1) / t); }
 
 // ---------------------------------------------------------------------------
 // Convolution 3x3, stride 1, zero padding 1: out = act(conv(in, w) + bias)
-// in [N][H][W][KIN], out [N][H][W][NOUT], w in the operand order of
-// k_prep_weights.
+// in [N][H][W][KIN], out [N][H][W][NOUT], w in the order of conv_weights.h.
 // With C0 > 0 the input is the concatenation the decoder convolves (skip
 // connection): channels [0, C0) are the nearest 2x upsampling of
 // low [N][H/2][W/2][C0], channels [C0, KIN) come from in [N][H][W][KIN - C0];
@@ -477,25 +475,18 @@ __global__ void k_adam(float* __restrict__ w, float* __restrict__ m, float* __re
 }
 
 // bf16 weight copies of one layer from the fp32 master [9][cin][cout], in the
-// order in which k_conv's lanes hold them: [K-step][16 outputs][lane][8], K =
-// (tap, input channel) padded with zeros to whole steps of 32. `wf`: the
-// layer itself; `wb`: its data gradient, taps mirrored, channels exchanged.
+// order of conv_weights.h. `wf`: the layer itself; `wb`, unless null: its data
+// gradient, taps mirrored, channels exchanged.
 __global__ void k_prep_weights(const float* __restrict__ w, int cin, int cout, uint16_t* __restrict__ wf,
                                uint16_t* __restrict__ wb)
 {
-    const int nf = conv_weights(cin, cout), nb = conv_weights(cout, cin);
+    const int nf = conv_weights(cin, cout), nb = wb ? conv_weights(cout, cin) : 0;
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if(t >= nf + nb) return;
     const bool back = t >= nf;
     const int e = back ? t - nf : t;
-    const int kin = back ? cout : cin, nt = (back ? cin : cout) / 16;
-    const int lane = (e >> 3) & 63, block = e >> 9;
-    const int k = 32 * (block / nt) + 8 * (lane >> 4) + (e & 7);
-    const int o = 16 * (block % nt) + (lane & 15);
-    const int tap = k / kin, c = k - (k / kin) * kin;
-    float v = 0.0f;
-    if(tap < 9) v = back ? w[((long)(8 - tap) * cin + o) * cout + c] : w[((long)tap * cin + c) * cout + o];
-    (back ? wb : wf)[e] = f2bf(v);
+    const int from = back ? conv_gradient_master_index(e, cin, cout) : conv_master_index(e, cin, cout);
+    (back ? wb : wf)[e] = f2bf(from >= 0 ? w[from] : 0.0f);
 }
 
 // Network input from a frame of the stochastic mode: noisy RGB (BASE),
@@ -688,7 +679,7 @@ Denoiser::Denoiser(uint32_t seed)
     check(hipMalloc(&adamM, numParams * 4));
     check(hipMalloc(&adamV, numParams * 4));
     check(hipMalloc(&wFwd, fwdOff * 2));
-    check(hipMalloc(&wBwd, bwdOff * 2));
+    if(kDenoiserBackwardEnabled) check(hipMalloc(&wBwd, bwdOff * 2));
     check(hipMemset(adamM, 0, numParams * 4));
     check(hipMemset(adamV, 0, numParams * 4));
     check(hipDeviceSynchronize()); // the fills are done before any stream's work reads them
@@ -724,9 +715,10 @@ Denoiser::~Denoiser()
 void Denoiser::prep_weights(hipStream_t s)
 {
     for(int l = 0; l < kNumLayers; ++l) {
-        const int n = conv_weights(kLayers[l].cin, kLayers[l].cout) + conv_weights(kLayers[l].cout, kLayers[l].cin);
-        k_prep_weights<<<grid_for(n, kThreads), kThreads, 0, s>>>(params + wOff[l], kLayers[l].cin, kLayers[l].cout,
-                                                                  wFwd + wFwdOff[l], wBwd + wBwdOff[l]);
+        const int cin = kLayers[l].cin, cout = kLayers[l].cout;
+        const int n = conv_weights(cin, cout) + (wBwd ? conv_weights(cout, cin) : 0);
+        k_prep_weights<<<grid_for(n, kThreads), kThreads, 0, s>>>(params + wOff[l], cin, cout, wFwd + wFwdOff[l],
+                                                                  wBwd ? wBwd + wBwdOff[l] : nullptr);
     }
     weightsReady = true;
 }

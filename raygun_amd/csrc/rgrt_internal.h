@@ -320,6 +320,12 @@ struct ShadeParams {
 // ---------------------------------------------------------------------------
 // Learned denoiser (denoise.hip)
 // ---------------------------------------------------------------------------
+// The backward pass (and so training) is switched off: its first GPU run
+// faulted in the weight-gradient kernel (an address beyond the legal range)
+// and no out-of-bounds access has been found in any of its kernels, so it
+// stays off the GPU until a cause is shown.
+constexpr bool kDenoiserBackwardEnabled = false;
+
 class Denoiser {
   public:
     static constexpr int kNumLayers = 11;
@@ -371,7 +377,7 @@ class Denoiser {
     size_t numParams = 0;
     size_t wOff[kNumLayers], bOff[kNumLayers], wFwdOff[kNumLayers], wBwdOff[kNumLayers];
     float *params = nullptr, *grads = nullptr, *adamM = nullptr, *adamV = nullptr;
-    uint16_t *wFwd = nullptr, *wBwd = nullptr;
+    uint16_t *wFwd = nullptr, *wBwd = nullptr; // wBwd: only where the backward pass is enabled
     bool weightsReady = false;
     bool paramsLoaded = false;
     uint32_t stepCount = 0;
