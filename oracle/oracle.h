@@ -58,6 +58,10 @@ int32_t orc_export_tlas(orc_scene* s, void* nodes, uint32_t* leafInstance);
  * not null, receive per-ray counts of visited BVH nodes / tested triangles. */
 int32_t orc_trace_rays(orc_scene* s, const float* rays, uint32_t n, uint32_t cullMask, void* hits, uint8_t* tie,
                        uint32_t* nodes, uint32_t* tris, int32_t threads);
+/* Entries a traversal with one stack for both levels holds at most on each
+ * ray's way: a bottom entry, the siblings of the nearest child at every level
+ * walked and an entry for the return from a BLAS. */
+int32_t orc_stack_depths(orc_scene* s, const float* rays, uint32_t n, uint32_t cullMask, uint32_t* depths, int32_t threads);
 /* Same queries by brute force in FP64 over every triangle of every instance. */
 int32_t orc_trace_rays_fp64(orc_scene* s, const float* rays, uint32_t n, uint32_t cullMask, double* t_out,
                             uint32_t* inst_out, uint32_t* prim_out, double* uv_out, int32_t threads);

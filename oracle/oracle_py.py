@@ -65,6 +65,8 @@ def lib():
         L.orc_export_tlas.argtypes = [P, P, P]
         L.orc_trace_rays.restype = i32
         L.orc_trace_rays.argtypes = [P, P, u32, u32, P, P, P, P, i32]
+        L.orc_stack_depths.restype = i32
+        L.orc_stack_depths.argtypes = [P, P, u32, u32, P, i32]
         L.orc_trace_rays_fp64.restype = i32
         L.orc_trace_rays_fp64.argtypes = [P, P, u32, u32, P, P, P, P, i32]
         L.orc_trace_rays_brute32.restype = i32
@@ -187,6 +189,14 @@ class OracleScene:
         if counts:
             return hits, tie.astype(bool), nodes, tris
         return hits, tie.astype(bool)
+
+    def stack_depths(self, rays, cull_mask=0xFF, threads=None):
+        """Entries a traversal with one stack for both levels holds at most, per ray."""
+        from raygun_amd.records import RAY
+        rays = np.ascontiguousarray(rays, RAY)
+        out = np.zeros(len(rays), np.uint32)
+        lib().orc_stack_depths(self.h, _p(rays), len(rays), cull_mask, _p(out), threads or default_threads())
+        return out
 
     def trace_rays_fp64(self, rays, cull_mask=0xFF, threads=None):
         from raygun_amd.records import RAY

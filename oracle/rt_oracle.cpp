@@ -885,6 +885,7 @@ struct Hit {
     bool tie = false;
     uint32_t nodes = 0, tris = 0;
     uint32_t instLeaves = 0, blasEntries = 0; // instance leaves reached, BLASes entered
+    uint32_t depth = 1; // most entries on one stack for both levels (orc_stack_depths)
 };
 
 constexpr float TIE_REL = 1e-6f;
@@ -964,7 +965,9 @@ bool trace_closest(const orc_scene& s, const float o[3], const float d[3], float
     while(tsp) {
         int32_t ref = tstack[--tsp];
         if(ref >= 0) {
+            const int before = tsp;
             visit(s.tlas.wideq, wr, ref, tstack, tsp);
+            if(tsp > before) h.depth = std::max(h.depth, 1u + (uint32_t)(tsp - 1)); // the nearest is walked, not stacked
             continue;
         }
         uint32_t ii = s.tlas.leafPrim[~ref];
@@ -975,6 +978,7 @@ bool trace_closest(const orc_scene& s, const float o[3], const float d[3], float
         const Blas& b = s.blas[ix.rec.blas];
         if(b.numFaces == 0) continue;
         h.blasEntries++;
+        h.depth = std::max(h.depth, 2u + (uint32_t)tsp);
         const float* w = ix.w2o;
         float oo[3], od[3];
         for(int row = 0; row < 3; ++row) {
@@ -989,7 +993,9 @@ bool trace_closest(const orc_scene& s, const float o[3], const float d[3], float
         while(bsp) {
             int32_t bref = bstack[--bsp];
             if(bref >= 0) {
+                const int before = bsp;
                 visit(b.bvh.wideq, r, bref, bstack, bsp);
+                if(bsp > before) h.depth = std::max(h.depth, 2u + (uint32_t)(tsp + bsp - 1));
                 continue;
             }
             uint32_t prim = b.bvh.leafPrim[~bref];
@@ -1982,6 +1988,17 @@ int32_t orc_trace_rays(orc_scene* s, const float* rays, uint32_t n, uint32_t cul
             if(nodes) nodes[i] = h.nodes;
             if(tris) tris[i] = h.tris;
         }
+    });
+    return 0;
+}
+
+int32_t orc_stack_depths(orc_scene* s, const float* rays, uint32_t n, uint32_t cullMask, uint32_t* depths, int32_t threads)
+{
+    parallel_rows(0, (int)n, threads, [&](int i, int) {
+        const float* r = rays + 8 * (size_t)i;
+        Hit h;
+        trace_closest(*s, r, r + 4, r[3], r[7], cullMask, h);
+        depths[i] = h.depth;
     });
     return 0;
 }

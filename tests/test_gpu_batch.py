@@ -38,6 +38,32 @@ def test_batched_frames_equal_sequential_frames(mode):
         b.close()
 
 
+def test_persistent_batch_with_sorted_queue_ends():
+    """A scene of more than 2^20 slots fills its queue from both ends, in a
+    persistent batch in one strip: beside a small scene that does not, the
+    frames are those of the scenes one by one."""
+    print("[case] persistent batch above 2^20 slots", flush=True)
+    big, small = (1100, 960), (96, 64)
+    work = []
+    for mode in (rgrt.BATCH_PERSISTENT, rgrt.BATCH_GRAPH_PER_SCENE):
+        w = batched.BatchWorkload(num_scenes=1, seed=11, lo=4_000, hi=4_000, resolutions=[small])
+        w.scenes.append(batched.BatchScene(1, 12, 4_000, big))
+        w.batch.close()
+        w.batch = rgrt.Batch([s.ctx for s in w.scenes], mode)
+        work.append(w)
+    a, b = work
+    try:
+        for f in range(2):
+            a.frame_batched(0.4 * f)
+            b.frame_sequential(0.4 * f)
+            for k, (sa, sb) in enumerate(zip(a.scenes, b.scenes)):
+                assert np.array_equal(sa.ctx.read_image(rgrt.IMAGE_FINAL), sb.ctx.read_image(rgrt.IMAGE_FINAL)), (f, k)
+            assert a.rays() == b.rays() > 1100 * 960
+    finally:
+        a.close()
+        b.close()
+
+
 @pytest.mark.parametrize("mode", [rgrt.BATCH_GRAPH_PER_SCENE, rgrt.BATCH_ONE_GRAPH, rgrt.BATCH_PERSISTENT])
 def test_batch_refuses_a_bad_scene_and_recovers(mode):
     print(f"[case] batch error path mode {mode}", flush=True)

@@ -47,3 +47,19 @@ def test_hits_do_not_depend_on_the_call_size(n):
             assert got["instance"][got["instance"] != 0xFFFFFFFF].max() < len(inst)
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("n", [1, 5000])
+def test_a_context_without_images_answers_ray_queries(n):
+    print(f"[case] rays without images {n}", flush=True)
+    setup = procgen.config2(64, 64, tris_per_mesh=500, num_instances=12)
+    ctx, inst = gpu_context(setup)
+    bare = ctx.shared(width=0, height=0)
+    try:
+        bare.build_tlas(inst)
+        rays = random_rays(n, 3, radius=70.0)
+        rays["tmax"] = 300.0
+        assert np.array_equal(bare.trace_rays(rays).view(np.uint8), ctx.trace_rays(rays).view(np.uint8))
+    finally:
+        bare.close()
+        ctx.close()

@@ -1,7 +1,10 @@
 """The traversal's stack past its LDS part: long thin triangles fanned about a
-line overlap in every box, so rays along it keep tens of entries waiting, in
-one and in two levels. Every distance equals, bit for bit, the oracle's brute
-force in 32 bits over all triangles with the same watertight test."""
+line overlap in every box, so rays along it keep more entries waiting than
+there are in LDS, in one and in two levels; the oracle's traversal counts them.
+Every distance equals, bit for bit, the oracle's brute force in 32 bits over
+all triangles with the same watertight test. Calls of few rays have a ray or a
+few per wave; above 32,768 the waves are full, and every second ray passes the
+fan's end with fewer entries, so a wave has lanes on both sides of the limit."""
 import numpy as np
 import pytest
 
@@ -10,6 +13,8 @@ from raygun_amd import rgrt
 from raygun_amd.records import INSTANCE, MATERIAL, NO_HIT, RAY, VERTEX
 
 pytestmark = pytest.mark.gpu
+
+LDS_ENTRIES = 16  # kLdsStack in trace.hip
 
 
 def fan(n, seed):
@@ -26,7 +31,7 @@ def fan(n, seed):
     return v, np.arange(3 * n, dtype=np.uint32)
 
 
-@pytest.mark.parametrize("tris,instances,rays", [(1, 1, 1), (2, 3, 63), (700, 1, 65), (700, 40, 1000)])
+@pytest.mark.parametrize("tris,instances,rays", [(1, 1, 1), (2, 3, 63), (700, 1, 65), (700, 40, 1000), (700, 2, 40_000)])
 def test_hits_with_entries_past_the_lds_stack(tris, instances, rays):
     print(f"[case] stack tris={tris} instances={instances}", flush=True)
     v, i = fan(tris, 3)
@@ -41,6 +46,8 @@ def test_hits_with_entries_past_the_lds_stack(tris, instances, rays):
     r["origin"] = np.stack([rng.uniform(-0.1, 0.1, rays), rng.uniform(-0.1, 0.1, rays), np.full(rays, -2.0)], 1)
     r["dir"] = np.stack([rng.normal(0, 0.01, rays), rng.normal(0, 0.01, rays), np.ones(rays)], 1)
     r["tmin"], r["tmax"] = 0.0, 100.0
+    if rays > 32_768:
+        r["origin"][1::2, 0] += 1.0
     ctx = rgrt.Context(16, 16)
     osc = oracle_py.OracleScene(v, i, np.zeros(0, MATERIAL))
     try:
@@ -49,6 +56,12 @@ def test_hits_with_entries_past_the_lds_stack(tris, instances, rays):
         ctx.build_tlas(inst)
         assert osc.build_blas(0, 0, tris) == inst["blas"][0]
         osc.build_tlas(inst)
+        depth = osc.stack_depths(r)
+        if tris > 2:
+            assert np.all(depth[::2] > LDS_ENTRIES)
+        if rays > 32_768:
+            spills = depth[:rays // 64 * 64].reshape(-1, 64) > LDS_ENTRIES
+            assert not np.any(np.all(spills, 1)) and np.median(depth[1::2]) > 4
         got = ctx.trace_rays(r)
         t, instance, _ = osc.trace_rays_brute32(r)
         hit = instance != NO_HIT
