@@ -967,14 +967,10 @@ __global__ __launch_bounds__(kDepthTopThreads) void k_wide_levels_top(const Node
     __shared__ uint32_t nextCount, subCount;
     if(threadIdx.x == 0) {
         subCount = 0;
-        frontA[0] = 0;
-        if(numInternal < kSubtree) { // the whole tree is one
-            subtrees[0] = make_uint2(0u, 0u);
-            subCount = 1;
-        }
+        frontA[0] = 0; // the root has more than kSubtree leaves (kCollapseOneBlock)
     }
     __syncthreads();
-    uint32_t count = numInternal < kSubtree ? 0u : 1u;
+    uint32_t count = 1;
     for(uint32_t d = 0; d < 128u && count > 0u; ++d) {
         if(threadIdx.x == 0) nextCount = 0;
         __threadfence_block();
@@ -1661,6 +1657,7 @@ __global__ void k_leaf_parents(const Node* __restrict__ nodes, uint32_t numInter
 // both take 150, for 1M triangles it is 1138 against 600 us (alone 2303
 // against 971; the numbering itself 1348 against 140).
 constexpr uint32_t kCollapseOneBlock = 32768;
+static_assert(kCollapseOneBlock >= (uint32_t)kSubtree, "k_wide_levels_top starts at a root above the subtrees");
 
 void LbvhBuilder::collapse(hipStream_t s, uint32_t n, const Node* nodes, Node4* wide, uint32_t* numWide)
 {

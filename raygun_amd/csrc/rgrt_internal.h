@@ -314,7 +314,7 @@ struct ShadeParams {
     int32_t keepAov;
     uint32_t sampling; // RGRT_SAMPLING_*
     uint32_t seed;
-    int32_t aheadOn; // shading passes may queue rays ahead (0: more slots than an entry can name)
+    int32_t aheadOn; // shading passes queue rays ahead (api.hip rays_ahead: few slots, one sample in each)
 };
 
 // ---------------------------------------------------------------------------
@@ -431,14 +431,12 @@ void launch_drain_multi(hipStream_t s, const ShadeParams* ps, const TraceScene* 
 // pixel (sample groups >= samples): the shading kernels then leave out the
 // start of a next sample.
 bool run_one_sample(const ShadeParams& p);
-void launch_trace_queue(hipStream_t s, const TraceScene& sc, const WavefrontState& st, int cur, uint32_t gridBlocks);
 // ahead: a traversal pass follows this shading pass (not the drain)
 void launch_shade(hipStream_t s, const ShadeParams& p, int cur, uint32_t gridBlocks, bool ahead);
 void launch_finalize_samples(hipStream_t s, const ShadeParams& p);
 void launch_drain(hipStream_t s, const ShadeParams& p, const TraceScene& sc, int cur, uint32_t gridBlocks, int32_t* spill);
 uint32_t drain_spill_words_per_thread();
 uint32_t drain_block_size();
-void launch_trace_rays(hipStream_t s, const TraceScene& sc, const rgrt_ray* rays, uint32_t n, uint32_t cullMask, rgrt_hit* hits);
 void launch_post(hipStream_t s, const Images& img, const rgrt_ubo& ubo, int useFxaa, hipEvent_t roughEnd);
 // rgba16f -> 8-bit RGBA / BGRA (optionally sRGB-encoded), 4 bytes per pixel
 void launch_to_rgba8(hipStream_t s, const uint16_t* src, uint8_t* dst, size_t npix, int bgra, int srgb);

@@ -52,8 +52,6 @@ struct BoxRay {
     float ix, iy, iz; // 1/d (zero components made finite)
 };
 
-__device__ __forceinline__ float pow2i(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
-
 // The hardware's three-operand maximum and minimum (fmaxf and fminf would
 // first quiet operands the compiler cannot prove quiet; the box test never
 // meets a NaN from finite rays, and one only culls or not).
