@@ -381,7 +381,8 @@ rgrt_status traversal_errors(rgrt_ctx* c)
 // bytes. The rays are read from, and hits and error word written to, pinned
 // memory of the context instead, with one wait: one ray 57 -> 35 us, 1,024
 // 97 -> 71, 4,096 123 -> 95 (hits through a device buffer and one more copy: 86
-// and 115).
+// and 115). It would go on: 16,384 rays 158 -> 124 us, 65,536 284 -> 246. The
+// limit is there for the memory, 208 KB of pinned memory in every context.
 constexpr uint32_t kPinnedRays = 4096;
 constexpr size_t kRayIoHits = kPinnedRays * sizeof(rgrt_ray), kRayIoError = kRayIoHits + kPinnedRays * sizeof(rgrt_hit);
 
@@ -445,13 +446,19 @@ void free_images(rgrt_ctx* c)
 
 // Whether a frame's shading passes queue reflection and refraction rays ahead
 // (wavefront.hip): it makes the chain of passes a third shorter, but the
-// shading kernel that takes such hits needs 155 VGPRs instead of 128. Small
+// shading kernel that takes such hits needs 160 VGPRs instead of 128. Small
 // frames wait on the chain; large ones, and several frames in flight, on the
-// work. Measured (pipelined): 640x360 0.587 -> 0.479 ms and with a rebuilt
-// mesh 0.635 -> 0.500, batches of 320x180 to 960x540 scenes 3.81 -> 3.39;
-// 960x540 over 3,000 instances 3.66 -> 3.89 and 1080p over 2M triangles 8.75
-// -> 9.8 ms. Slots that run several samples one after another keep the plain
-// kernels.
+// work. The line lies where frames in flight stop gaining. Without and with
+// rays ahead, us per frame, one sphere (depth 1) | 32 instances (depth 4):
+//   slots    one at a time           2 in flight
+//    57,600   449, 357 | 1916, 1619   272, 232 |  965, 825
+//   230,400   518, 434 | 2055, 1988   306, 276 | 1073, 1029
+//   291,600   554, 500 | 2174, 2088   327, 333 | 1123, 1076
+//   518,400   654, 643 | 2232, 2196   432, 485 | 1200, 1161
+// 960x540 (518,400) over 3,000 instances takes 3.66 and 3.89 ms, 1080p over 2M
+// triangles 8.75 and 9.8. The number in flight is not known to a context, so
+// the rule is the slot count. Slots that run several samples one after another
+// keep the plain kernels.
 constexpr uint32_t kAheadSlots = 300000;
 static_assert(kAheadSlots <= kAheadMaxSlots, "a queue entry names its slot");
 

@@ -17,9 +17,10 @@ constexpr int kSpill = 368; // with the 16 LDS entries: the 382-entry worst case
 // the rays queued ahead -> the frames that will need their hits. Waves fetch
 // 64 rays at a time from a global counter (persistent grid).
 // Waves per SIMD the traversal pass is compiled for: the register budget is
-// 512 / waves VGPRs, its loop needs 94. At 6 waves (80, seven spilled in the
-// loop) 3,000 small instances take 3.62 ms against 3.43 at 5, a 640x360 frame
-// 0.465 against 0.447, larger frames the same.
+// 512 / waves VGPRs, its loop needs 94. At 6 waves (80, twelve spilled) 3,000
+// small instances take 3.52 ms against 3.32 at 5, a 640x360 frame 0.466 against
+// 0.446, 1080p over 2M triangles 7.47 against 7.17, 4K at 4 samples 86.2
+// against 84.3.
 #ifndef RGRT_TRACE_WAVES
 #define RGRT_TRACE_WAVES 5
 #endif

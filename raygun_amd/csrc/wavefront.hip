@@ -46,6 +46,11 @@ constexpr int kShadeBlock = 256;
 
 // Minimum waves per SIMD the shading kernels are compiled for (the register
 // budget is then 512 / waves VGPRs; what does not fit spills to scratch).
+// The variants that may start a slot's next sample take what they need: 154
+// (3 waves) and 181 VGPRs (the drain, 2 waves). With the drain at 3 waves, 4
+// samples one after another take 4.49 against 4.34 ms at 640x360 and 7.85
+// against 8.10 at 1920x1080, in a persistent batch of eight scenes 9.73
+// against 9.54.
 #ifndef RGRT_SHADE_WAVES
 #define RGRT_SHADE_WAVES 1
 #endif
@@ -60,14 +65,16 @@ constexpr int kShadeBlock = 256;
 #define RGRT_SHADE1_WAVES 4
 #endif
 // The drain variant for one sample per slot (no next-sample start) fits in
-// 143 VGPRs (3 waves); compiled for 4 waves it spills 12 VGPRs and runs
-// faster (config 2 at 1080p: 1.58-1.60 against 1.69-1.82 ms). At 5 waves it
-// spills 55 inside the traversal loop: 5.60 against 5.34-5.36 ms per
-// frame with four frames in flight.
+// 154 VGPRs (3 waves); compiled for 4 waves it spills 20 and the frames are
+// faster: 1080p over 2M triangles 7.16 against 7.35 ms, 4K at 4 samples 83.5
+// against 86.0, 960x540 over 3,000 instances 3.32 against 3.37 (1283x721 at 2
+// samples 9.51 against 9.42).
 #ifndef RGRT_DRAIN1_WAVES
 #define RGRT_DRAIN1_WAVES 4
 #endif
 
+// With rays ahead: 160 VGPRs (shading), and 178 for the drain, of which it
+// spills 7 at 3 waves.
 #ifndef RGRT_SHADE_AHEAD_WAVES
 #define RGRT_SHADE_AHEAD_WAVES 3
 #endif
