@@ -37,17 +37,17 @@ RAY_BYTES = 40    # queue entry: origin, tmin, dir, tmax, pixel, flags
 HIT_BYTES = 20    # t, u, v, instance, primitive
 GATHER_BYTES = 184  # closest-hit gathers: 12 B indices + 96 B vertices + 64 B material + 12 B offsets
 # config 5 (4 samples per pixel, depth 6): far longer per-pixel ray chains
-CONFIG5_CANDIDATES = {"wavefrontPasses": [24, 32, 48, 64], "traceBlocksPerCU": [3, 4, 5],
+CONFIG5_CANDIDATES = {"wavefrontPasses": [24, 32, 48, 64], "traceBlocksPerCU": [4, 5],
                       "drainBlocksPerCU": [2, 4, 8]}
 # launch shapes the autotuner tries for the headline pipeline (coordinate descent)
-TUNE_CANDIDATES = {"wavefrontPasses": [6, 8, 10, 12, 14], "traceBlocksPerCU": [3, 4, 5],
+TUNE_CANDIDATES = {"wavefrontPasses": [6, 8, 10, 12, 14], "traceBlocksPerCU": [4, 5],
                    "drainBlocksPerCU": [2, 4, 8], "shadeBlocksPerCU": [4, 8, 12], "frameBands": [1, 2]}
 # One frame at a time the recursion tail is not hidden by the next frame:
 # the frame traced in bands on separate streams (so one band's sparse last
 # passes overlap another's work), fewer wavefront passes and a larger drain
 # grid pay off.
 ONE_FRAME_CANDIDATES = {"frameBands": [1, 2, 3, 4], "wavefrontPasses": [3, 4, 5, 6, 8, 10],
-                        "drainBlocksPerCU": [2, 3, 4], "traceBlocksPerCU": [3, 4, 5], "shadeBlocksPerCU": [4, 8, 12]}
+                        "drainBlocksPerCU": [2, 3, 4], "traceBlocksPerCU": [4, 5], "shadeBlocksPerCU": [4, 8, 12]}
 
 
 def log(msg):
@@ -683,7 +683,7 @@ def bench_batched(num_scenes, frames):
     log(f"[bench] batched workload: {num_scenes} scenes, {sum(w.info['triangles'])} triangles, "
         f"{w.info['pixels']} pixels, built in {time.time() - t0:.1f}s")
     try:
-        cand = {"wavefrontPasses": [2, 4, 6, 8], "traceBlocksPerCU": [3, 4, 5]}
+        cand = {"wavefrontPasses": [2, 4, 6, 8], "traceBlocksPerCU": [4, 5]}
         t1 = time.time()
         tunings = []
         for sc in w.scenes:

@@ -15,7 +15,7 @@ from .hiptime import HipEvents, time_ms
 
 CANDIDATES = {
     "wavefrontPasses": [2, 4, 6, 8, 12],
-    "traceBlocksPerCU": [3, 4, 5],
+    "traceBlocksPerCU": [4, 5],
     "shadeBlocksPerCU": [4, 8, 12],
     "drainBlocksPerCU": [2, 4, 8],
     "hostLag": [1, 2, 4],

@@ -72,7 +72,7 @@ inline uint32_t grid_for(uint64_t n, uint32_t t) { return (uint32_t)((n + t - 1)
 // and its image kernels 786 -> 430 us. The waves a SIMD holds (seven at 16
 // channels, four at 48 to 16 and 32 to 64; 96 to 32 and 64 to 64, with 43 and
 // 51 KB of LDS a workgroup, three and two) hide a tile's copy
-// behind the products of the others; with two (all steps' operands loaded
+// behind the products of the others; with two everywhere (all steps' operands loaded
 // ahead) the same code took as long as the loads from memory had.
 // ---------------------------------------------------------------------------
 template <int KIN, int NOUT, int C0 = 0>
