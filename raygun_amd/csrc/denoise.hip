@@ -67,9 +67,9 @@ inline uint32_t grid_for(uint64_t n, uint32_t t) { return (uint32_t)((n + t - 1)
 // The weights are the first operand: a lane then holds four consecutive
 // channels of one pixel, so that a strip of 16 pixels is stored whole.
 // Measured at 1920 x 1080, operands loaded from memory for each tap -> this
-// kernel: 16 to 16 channels 52 -> 33 us (133 MB, 4.0 TB/s), 48 to 16 156 -> 62,
-// 96 to 32 104 -> 42, 32 to 32 45 -> 22, 64 to 64 64 -> 24; the whole network
-// and its image kernels 786 -> 430 us. The waves a SIMD holds (seven at 16
+// kernel: 16 to 16 channels 52 -> 35 us (159 MB by the counters, 4.6 TB/s), 48 to
+// 16 156 -> 64, 96 to 32 104 -> 43, 32 to 32 45 -> 23, 64 to 64 64 -> 25; the whole
+// network and its image kernels 786 -> 437 us. The waves a SIMD holds (seven at 16
 // channels, four at 48 to 16 and 32 to 64; 96 to 32 and 64 to 64, with 43 and
 // 51 KB of LDS a workgroup, three and two) hide a tile's copy
 // behind the products of the others; with two everywhere (all steps' operands loaded
