@@ -550,7 +550,7 @@ rgrt_status rgrt_get_tuning(rgrt_ctx* ctx, rgrt_tuning* t);
  * them are traced side by side in separate wavefront slots; each sample's
  * record is kept and the records are summed in sample order afterwards, so
  * the images equal those of one sample at a time bit for bit. 0 (default):
- * as many as fit 2^25 slots (~1.26 KB of device memory each); 1: one
+ * as many as fit 2^25 slots (~0.8 KB of device memory each); 1: one
  * sample at a time; at most 32. */
 rgrt_status rgrt_set_sample_groups(rgrt_ctx* ctx, uint32_t maxGroups);
 
